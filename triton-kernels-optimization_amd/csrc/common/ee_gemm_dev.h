@@ -198,6 +198,26 @@ EE_DEV void store_row16(uint16_t* dst, const u32x4& v, bool full) {
     }
 }
 
+// XCD x = blockIdx % 8 takes a contiguous eighth of a list of n tiles; *i, the workgroup's
+// index on its XCD, becomes an index into the list (true), or is moved past that eighth.
+EE_DEV bool xcd_share(int n, int& i) {
+    const int x = (int)blockIdx.x & 7, q = n >> 3, r = n & 7, own = q + (x < r);
+    if (i < own) {
+        i += x * q + min(x, r);
+        return true;
+    }
+    i -= own;
+    return false;
+}
+
+// i / t for tile indices (0 <= i < 2^20, t > 0; a list of that many tiles would be a C of terabytes):
+// (i + 0.5) / t is at least 0.5 / t from an integer and the product below within i / t * 2^-22 of it.  A
+// divide by a count from memory is on the kernel's critical path: an integer division there
+// (~40 dependent instructions) cost 0.4 us per launch.
+EE_DEV int tile_div(int i, int t) {
+    return __builtin_amdgcn_readfirstlane((int)(((float)i + 0.5f) * __builtin_amdgcn_rcpf((float)t)));
+}
+
 // Tile order and the deal of tiles to workgroups (shared by the plain and the
 // routed persistent kernels).  Logical tiles a = 0 .. nA-1 (the 1-byte-operand
 // tiles) are ordered in bands of 8 M-tiles walked along N, so 32 consecutive

@@ -1651,10 +1651,14 @@ EE_GEMM_ENTRY(eek_gemm_w8a16, body_w8a16)
 
 // The routed linear's three tier GEMMs in one launch.  Tier t owns partition
 // slots [off_t, off_t + counts[t]) (off_t = counts[0] + ... + counts[t-1]) and
-// the ceil(counts[t] / 128) M-tile indices after those of the lower tiers, so
-// an M-tile never mixes tiers; workgroups past the last tile exit at once.
-// The grid holds r.mt_max = ceil(M / 128) + 2 M-tile slots (the sum of the
-// three ceilings is at most that) times ceil(N / 128) N-tiles.
+// its own ceil(counts[t] / 128) M-tiles, so a tile never mixes tiers.  The grid holds
+// r.mt_max = ceil(M / 128) + 2 M-tiles per N-tile (the sum of the three ceilings is at
+// most that); the tiles that exist are counted here, from the device's counts: every XCD
+// takes an eighth of each tier's list, the FP16 tiles (twice a 1-byte tile's time) first,
+// and the surplus workgroups come last.  (They used to be every mt_max-th one: with half the
+// slots empty the CUs of a round were dealt two tiles or none.  Measured, us before / now: 200 x 2048
+// x 11264 SwiGLU, 20/40/40 % tiers 42.9 / 26.1, 512 rows 44.4 / 37.0, 300 x 4096 x 14336 98% FP8 92.7 /
+// 64.7, 8 x 2048 x 32000 INT8 32 / 15.5; grids of one round within 0.4 us.)
 // FP16 halves (r.f16_half_cus > 0, no SwiGLU): an FP16 tile costs two 1-byte
 // tiles, so the FP16 tier takes two M-tile indices per M-tile, one per 128 x 64
 // column half (mt_max then counts them: at most 2 ceil(M / 128) + 2), where the
@@ -1672,26 +1676,33 @@ EE_DEV void gemm_routed(const EeRoutedGemmArgs& r) {
     const int T0 = (counts[0] + BM - 1) / BM;
     const int T1 = (counts[1] + BM - 1) / BM;
     const int T2 = (counts[2] + BM - 1) / BM;
-    int tm, tn;
-    tile_of((int)blockIdx.x, (int)gridDim.x, r.mt_max, tm, tn);
+    const int nN = (r.t[2].N + BN - 1) / BN;
+    const int wf = (T0 + T1 + T2) * nN, wh = (T0 + T1 + 2 * T2) * nN, cus = r.f16_half_cus;
+    const bool halves = SW == 0 && cus > 0 && T2 > 0 && (wh <= cus || (wf > cus && wf <= 2 * cus));
+    int i = (int)blockIdx.x >> 3;
     if constexpr (SW == 0) {
-        const int nN = (r.t[2].N + BN - 1) / BN;
-        const int wf = (T0 + T1 + T2) * nN, wh = (T0 + T1 + 2 * T2) * nN, cus = r.f16_half_cus;
-        if (cus > 0 && T2 > 0 && (wh <= cus || (wf > cus && wf <= 2 * cus)) && tm >= T0 + T1) {
-            const int v = tm - T0 - T1;
-            if (v < 2 * T2) gemm_tile<EE_GEMM_F16, 0, 64>(r.t[2], v >> 1, 2 * tn + (v & 1), smem);
-            return;
+        if (halves) {
+            if (xcd_share(2 * T2 * nN, i)) {
+                const int tn = tile_div(i, 2 * T2), v = i - tn * 2 * T2;
+                gemm_tile<EE_GEMM_F16, 0, 64>(r.t[2], v >> 1, 2 * tn + (v & 1), smem);
+                return;
+            }
         }
     }
-    if (tm < T0) gemm_tile<EE_GEMM_I8, SW>(r.t[0], tm, tn, smem);
-    else if (tm < T0 + T1) gemm_tile<EE_GEMM_F8, SW>(r.t[1], tm - T0, tn, smem);
-    else if (tm < T0 + T1 + T2) {
+    if (!halves && xcd_share(T2 * nN, i)) {
+        const int tn = tile_div(i, T2);
         if (r.f16_w8) {
             Gemm8<EE_GEMM_F16, SW> k(r.t[2], smem);
-            k.run(tm - T0 - T1, tn);
+            k.run(i - tn * T2, tn);
         } else {
-            gemm_tile<EE_GEMM_F16, SW>(r.t[2], tm - T0 - T1, tn, smem);
+            gemm_tile<EE_GEMM_F16, SW>(r.t[2], i - tn * T2, tn, smem);
         }
+    } else if (xcd_share(T1 * nN, i)) {
+        const int tn = tile_div(i, T1);
+        gemm_tile<EE_GEMM_F8, SW>(r.t[1], i - tn * T1, tn, smem);
+    } else if (xcd_share(T0 * nN, i)) {
+        const int tn = tile_div(i, T0);
+        gemm_tile<EE_GEMM_I8, SW>(r.t[0], i - tn * T0, tn, smem);
     }
 }
 extern "C" __global__ void __launch_bounds__(GEMM_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))

@@ -931,11 +931,11 @@ static int routed_impl(ee_engine* eng, const void* x, int64_t ld_x, int32_t M, i
         // the whole-tile grid takes one to two rounds (decided in the kernel from the
         // tier counts): possible only where one M-tile per 128 rows takes at most two
         // rounds.  The grid then holds the halves' M-tile slots too.
-        int64_t grid = pg > 0 ? pg : slots;
+        int64_t grid = pg > 0 ? pg : slots + 24;         // (xcd_share rounds each tier's list up to 8)
         if (pg == 0 && !sw && !ra.f16_w8 && cdiv(M, 128) * cdiv(N, 128) <= 2 * (int64_t)eng->cus) {
             ra.mt_max = (int32_t)(2 * cdiv(M, 128) + 2);
             ra.f16_half_cus = eng->cus;
-            grid = (int64_t)ra.mt_max * cdiv(N, 128);
+            grid = (int64_t)ra.mt_max * cdiv(N, 128) + 24;
         }
         std::string rname = pg > 0 ? "eek_gemm_routed_persist" : "eek_gemm_routed";
         if (sw) rname += "_swiglu";
