@@ -354,6 +354,11 @@ int ee_routed_linear_swiglu(ee_engine* eng, const void* x, int64_t ld_x, int32_t
                             const void* b_f16, const float* b_scale, void* act, int64_t ld_act, void* ws_codes,
                             float* ws_scale, ee_stream_t stream);
 
+/* Compute waves per tile if ee_gemm / ee_gemm_swiglu of this kind and shape (un-routed) runs the
+ * few-rows kernels (64-row tiles), 0 if it runs the larger tiles.  Where EE_GEMM_W8A16 runs
+ * them, its bits are EE_GEMM_F16's on ee_pack_b_f16's weights, from half the weight bytes. */
+int ee_gemm_small_waves(const ee_engine* eng, int32_t kind, int64_t M, int64_t N, int64_t K, int32_t swiglu);
+
 /* ---- allocation-free routed linear ----------------------------------------
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that

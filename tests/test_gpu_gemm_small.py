@@ -1,0 +1,134 @@
+"""The few-rows GEMM kernels (eek_gemm_m64w*, engine option gemm_small) against the
+larger tiles' bits: every tier sums K in the same order, so plain, SwiGLU, W8A16-from-codes
+and routed outputs are bit-identical, and INT8 also equals the oracle."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def ee():
+    import entropy_engine
+    yield entropy_engine
+    _opt(0)
+
+
+def _opt(v):
+    from entropy_engine import _lib
+    _lib.check(_lib.lib().ee_engine_set_option(_lib.engine(), b"gemm_small", v))
+
+
+def _last_kernel():
+    from entropy_engine import _lib
+    return _lib.lib().ee_last_kernel().decode()
+
+
+def _bits(t):
+    torch.cuda.synchronize()
+    return t.view(torch.int16)
+
+
+def _weight(ee, N, K, seed=0):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).half()
+    codes, scale = ee.quantize_weight_codes(w)
+    return ee.PackedWeight(codes, scale).materialize(), g
+
+
+# K: one stage up to several passes over the register ring, with partial chunks and passes
+SHAPES = [(1, 128, 4), (8, 256, 64), (9, 1152, 36), (16, 2176, 520), (17, 1024, 132), (32, 4096, 96), (33, 1920, 260),
+          (64, 640, 128), (65, 2048, 68), (130, 1408, 192), (300, 384, 64)]
+
+
+@pytest.mark.parametrize("cols", [16, 32, 64])
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_small_gemm_bits(ee, M, K, N, cols):
+    pw, g = _weight(ee, N, K, seed=M + N)
+    x = torch.randn(M, K + 16, generator=g, device="cuda").half()[:, :K]     # a row stride of its own
+    x[0] *= 30.0
+    i8, f8 = ee.quantize_activations(x, "dispatcher"), ee.quantize_activations(x, "fp8")
+    calls = [("int8", i8[0], pw.i8, i8[1], pw.scale), ("fp8", f8[0], pw.f8, f8[1], pw.scale),
+             ("fp16", x, pw.f16, None, None)]
+    for kind, a, b, sa, sb in calls:
+        _opt(1)
+        ref = ee.gemm(kind, a, b, sa, sb)
+        assert "m64" not in _last_kernel()
+        _opt(cols)
+        assert torch.equal(_bits(ee.gemm(kind, a, b, sa, sb)), _bits(ref)), kind
+        assert "m64w" in _last_kernel()
+        if kind == "fp16":
+            assert torch.equal(_bits(ee.gemm("w8a16", x, pw.i8, None, pw.scale)), _bits(ref)), "w8a16"
+            assert "m64w" in _last_kernel()
+
+
+@pytest.mark.parametrize("cols", [16, 32])
+@pytest.mark.parametrize("M,K,F", [(1, 128, 32), (8, 2048, 352), (20, 640, 96), (40, 1152, 64), (70, 512, 160)])
+def test_small_gemm_swiglu_bits(ee, M, K, F, cols):
+    pw, g = _weight(ee, 2 * F, K, seed=M)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    i8, f8 = ee.quantize_activations(x, "dispatcher"), ee.quantize_activations(x, "fp8")
+    for kind, a, b, sa, sb in [("int8", i8[0], pw.i8, i8[1], pw.scale), ("fp8", f8[0], pw.f8, f8[1], pw.scale),
+                               ("fp16", x, pw.f16, None, None)]:
+        _opt(1)
+        ref = ee.gemm(kind, a, b, sa, sb, swiglu=True)
+        _opt(cols)
+        assert torch.equal(_bits(ee.gemm(kind, a, b, sa, sb, swiglu=True)), _bits(ref)), kind
+        if kind == "fp16":
+            assert torch.equal(_bits(ee.gemm("w8a16", x, pw.i8, None, pw.scale, swiglu=True)), _bits(ref)), "w8a16"
+
+
+def test_small_gemm_int8_accumulators_and_oracle(ee, orc):
+    rng = np.random.default_rng(3)
+    M, K, N = 21, 1280, 100
+    a = rng.integers(-127, 128, (M, K), dtype=np.int8)
+    b = rng.integers(-127, 128, (N, K), dtype=np.int8)
+    sa, sb = rng.random(M, dtype=np.float32) + 0.1, rng.random(N, dtype=np.float32) * 1e-3
+    acc = torch.zeros((M, N), dtype=torch.int32, device="cuda")
+    _opt(16)
+    c = ee.gemm("int8", *(torch.from_numpy(t).cuda() for t in (a, b, sa, sb)), acc_out=acc)
+    ref = a.astype(np.int64) @ b.astype(np.int64).T
+    assert np.array_equal(acc.cpu().numpy(), ref)
+    out = ((ref.astype(np.float32) * sa[:, None]) * sb[None, :]).astype(np.float16)
+    assert np.array_equal(c.cpu().numpy().view(np.uint16), out.view(np.uint16))
+
+
+# rows of the three tiers: empty tiers, edges of the 16- and 64-row groups, several M-tiles
+@pytest.mark.parametrize("counts", [(1, 0, 0), (0, 1, 0), (0, 0, 1), (3, 4, 1), (16, 17, 33), (64, 0, 65), (5, 130, 20)])
+@pytest.mark.parametrize("K,N,sw", [(1024, 512, False), (2048, 260, False), (512, 192, True)])
+def test_small_routed_bits(ee, counts, K, N, sw):
+    M = sum(counts)
+    pw, g = _weight(ee, N, K, seed=M)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    h = torch.cat([torch.full((c,), t + 1.0) for t, c in enumerate(counts)])[torch.randperm(M)].cuda()
+    _, idx, cnt = ee.route(h, 1.5, 2.5)
+    _opt(1)
+    ref = ee.routed_linear(x, pw, idx, cnt, swiglu=sw)
+    assert "m64" not in _last_kernel()
+    for cols in (16, 32):
+        _opt(cols)
+        out = torch.full_like(ref, float("nan"))
+        ee.routed_linear(x, pw, idx, cnt, out=out, swiglu=sw)
+        assert "m64w" in _last_kernel()
+        assert torch.equal(_bits(out), _bits(ref))
+
+
+def test_small_gemm_choice(ee):
+    """Decode shapes take the small tiles, the headline shape does not; W8A16 from the codes
+    gives the FP16 tier's bits through the public call."""
+    from entropy_engine import _lib
+    L, e = _lib.lib(), _lib.engine()
+    for kind in range(4):
+        assert L.ee_gemm_small_waves(e, kind, 4, 4096, 4096, 0) > 0
+        assert L.ee_gemm_small_waves(e, kind, 1024, 4096, 4096, 0) == 0
+        assert L.ee_gemm_small_waves(e, kind, 4, 4096, 4104, 0) == 0        # K of whole 128-byte stages only
+    pw, g = _weight(ee, 1000, 1024)
+    x = torch.randn(5, 1024, generator=g, device="cuda").half()
+    lin = torch.nn.Linear(1024, 1000, bias=False, device="cuda", dtype=torch.float16)
+    layer = ee.EntropyDispatchedLinear.from_linear(lin)
+    y = layer(x)
+    assert "w8a16" in _last_kernel()
+    _opt(1)
+    assert torch.equal(_bits(y), _bits(layer(x)))

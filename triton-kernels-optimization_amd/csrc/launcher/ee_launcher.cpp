@@ -485,6 +485,9 @@ EE_EXPORT int ee_engine_set_option(ee_engine* eng, const char* key, int64_t valu
     } else if (k == "gemm_tile_n") {
         if (value != 0 && value != 128 && value != 256)
             return fail(EE_ERR_INVALID_ARG, k + " must be 0 (auto), 128 or 256");
+    } else if (k == "gemm_small") {
+        if (value != 0 && value != 1 && value != 16 && value != 32 && value != 64)
+            return fail(EE_ERR_INVALID_ARG, k + " must be 0 (auto), 1 (off), 16, 32 or 64");
     } else if (k == "gemm_waves") {
         if (value != 0 && value != 4 && value != 8)
             return fail(EE_ERR_INVALID_ARG, k + " must be 0 (auto), 4 or 8");
@@ -628,6 +631,72 @@ EE_EXPORT int ee_pack_b_f16(ee_engine* eng, const int8_t* codes_nk, const float*
     return launch(eng, "eek_pack_b_f16", g > 16384 ? 16384 : g, 1, EE_BLOCK, a, stream);
 }
 
+// ---- small GEMMs (gemm_small.hip): 64-row tiles, one column group of 16 (FP8: 32) per
+// compute wave, twice that with SwiGLU (gate and up).  SwiGLU has 1 and 2 waves only.
+static int64_t small_cols(int waves, int sw, bool f8) { return (int64_t)waves * (f8 ? 32 : 16) * (sw ? 2 : 1); }
+
+// Option "gemm_small": 0 auto, 1 off, 16 / 32 / 64 = 1 / 2 / 4 waves forced.  Returns the forced
+// waves, 0 for off (also where an option names another GEMM kernel), -1 for the automatic choice.
+static int small_forced(const ee_engine* e, int sw) {
+    const int64_t o = opt(e, "gemm_small");
+    if (o > 1) return (int)std::min<int64_t>(o / 16, sw ? 2 : 4);
+    if (o == 1 || opt(e, "gemm_variant") || opt(e, "gemm_persist") || opt(e, "gemm_tile") || opt(e, "gemm_waves") ||
+        opt(e, "gemm_tile_n"))
+        return 0;
+    return -1;
+}
+
+// Compute waves of an un-routed small GEMM, or 0 where the larger tiles are faster.
+// Both kinds of kernel are bound by the operand bytes a CU pulls through its L1 (the number of
+// requests it holds open), so the rule compares those: per K element of one round, rows * ea + columns
+// * eb bytes per workgroup, rounds = workgroups per CU rounded up; the 128 x 128 tile counts its
+// distinct rows.  The small tiles win by more than bytes (several workgroups per CU, no
+// padding) up to ~0.6 of the large tile's bytes, 0.75 at up to 32 rows.  Measured (us, large
+// against small tile; weights rotating through the Infinity Cache):
+//   INT8 K 4096, N 4096: M 4 13.8 / 5.5, M 64 15.0 / 9.1 (0.42), M 256 15.9 / 14.0 (0.50), M 512 16.3 /
+//     24.4 (1.0); N 14336: M 16 14.2 / 12.0 (0.56), M 64 15.4 / 16.9 (0.67), M 128 16.6 / 27.5 (0.87)
+//   FP8 K 4096, N 4096: M 4 13.3 / 8.4 (0.48), M 128 15.5 / 11.4 (0.38); N 14336: M 32 17.2 / 15.2 (0.6)
+//   FP16 against W8A16 codes, K 4096, N 4096: M 4 22.2 / 9.2, M 256 25.1 / 16.4 (0.38); N 14336: M 4
+//     35.3 / 12.9 (0.36), M 128 45.7 / 33.0 (0.75), M 256 47.3 / 62.2 (1.5)
+// W8A16 (int8 codes) also reads half the weight bytes, which counts by itself once the fp16
+// weights leave no room in the Infinity Cache for anything else: N K >= 32 Mi, up to 1.0.
+static int small_waves(const ee_engine* e, int32_t kind, int64_t M, int64_t N, int64_t K, int sw) {
+    const int f = small_forced(e, sw);
+    if (f >= 0) return f;
+    const bool f8 = kind == EE_GEMM_F8;
+    const int ea = kind == EE_GEMM_F16 || kind == EE_GEMM_W8A16 ? 2 : 1, eb = kind == EE_GEMM_F16 ? 2 : 1;
+    const int64_t r = f8 ? 32 : 16, rows = std::min<int64_t>(64, cdiv(M, r) * r), cu = std::max(1, e->cus);
+    const int64_t large = cdiv(cdiv(M, 128) * cdiv(N, 128), cu) * (std::min<int64_t>(M, 128) + 128) * ea;
+    int best = 0;
+    int64_t cost = 0;
+    for (int w = 1; w <= (sw ? 2 : 4); w *= 2) {
+        const int64_t c = small_cols(w, sw, f8), n = cdiv(cdiv(M, 64) * cdiv(N, c), cu) * (rows * ea + c * eb);
+        if (best == 0 || n < cost) {
+            best = w;
+            cost = n;
+        }
+    }
+    const int64_t pct = kind == EE_GEMM_W8A16 && N * K >= (int64_t(32) << 20) ? 100 : M <= 32 ? 75 : 60;
+    return cost * 100 <= large * pct ? best : 0;
+}
+
+// Compute waves of a routed small GEMM, or 0.  The tiers' row counts are on the device; about two M-tiles
+// more than the rows fill are taken to exist.  Measured on 20/40/40 and 1/98/1 % tiers (us, 128-tile
+// routed grid against this one): 8 x 4096 x 4096 19.9 / 12.6, 8 x 2048 x 32000 63 / 43, 64 x 4096 x 14336 54 /
+// 39, 128 x 2048 x 2560 12.3 / 10.7, 128 x 4096 x 14336 57 / 46, 300 x 5632 x 2048 27.1 / 19.4,
+// 300 x 2048 x 2048 13.0 / 10.8; slower at 512 x 2048 x 2048 (13.4 / 14.7), 200 x 4096 x 4096 (20.8 / 22.7),
+// 200 x 4096 x 14336 (58 / 72).  SwiGLU N 11264, K 2048: M 8 25.7 / 22.0, M 64 25.2 / 22.4, M 128 26.0 / 29.6.
+// One wave per tile with SwiGLU (98% FP8 rows, M 8: 11.1 us against 15.3 with two) and while that gives at most
+// ~3 workgroups per CU, else two; `dense`: past 4 workgroups per CU of two, the form with half the LDS.
+static int small_routed_waves(const ee_engine* e, int64_t M, int64_t N, int sw, bool& dense) {
+    const int f = small_forced(e, sw);
+    const int64_t mt = cdiv(M, 64) + 2, cu = std::max(1, e->cus), n2 = mt * cdiv(N, 32);
+    dense = !sw && n2 > 4 * cu;
+    if (f >= 0) return std::min(f, sw ? 1 : 2);
+    if (M > (sw ? 64 : 128) && (sw || n2 > 2 * cu)) return 0;
+    return sw || mt * cdiv(N, 16) * 8 <= 25 * cu ? 1 : 2;
+}
+
 // sw = 1: SwiGLU epilogue (b_nk gate|up interleaved in blocks of 32 rows; c is act [M, N/2]).
 static int gemm_impl(ee_engine* eng, int32_t kind, const void* a, int64_t lda, const void* b_nk, int64_t ldb,
                      void* c, int64_t ldc, const float* a_scale, const float* b_scale, int32_t M, int32_t N,
@@ -659,6 +728,11 @@ static int gemm_impl(ee_engine* eng, int32_t kind, const void* a, int64_t lda, c
         if (M == 0) return EE_OK;
         EeGemmArgs g{a, b_nk, (uint16_t*)c, nullptr, nullptr, b_scale, a_idx, c_idx, counts, lda, ldb, ldc,
                      M, N, K, counts ? tier : 0, sw};
+        if (const int t = counts == nullptr && K % 128 == 0 ? small_waves(eng, kind, M, N, K, sw) : 0) {
+            const std::string name = "eek_gemm_m64w" + std::to_string(t) + "_w8a16" + (sw ? "_swiglu" : "");
+            const Kernel* k = find_kernel(eng, name);
+            return launch(eng, name, cdiv(M, 64) * cdiv(N, small_cols(t, sw, false)), 1, k ? k->block : 64, g, stream);
+        }
         // The four-wave 256-row tiles (eek_gemm4w[n128]_w8a16) wherever EE_GEMM_F16 on
         // eek_pack_b_f16's weights would run eek_gemm4w[n128]_f16 (the conditions
         // below): the same MFMAs on the same weight values in the same K order, so
@@ -712,6 +786,12 @@ static int gemm_impl(ee_engine* eng, int32_t kind, const void* a, int64_t lda, c
     if (M == 0) return EE_OK;
     EeGemmArgs g{a, b_nk, (uint16_t*)c, acc_out, a_scale, b_scale, a_idx, c_idx, counts, lda, ldb, ldc,
                  M, N, K, counts ? tier : 0, sw};
+    if (const int t = counts == nullptr && (K * esz) % 128 == 0 ? small_waves(eng, kind, M, N, K, sw) : 0) {
+        static const char* names[3] = {"_i8", "_f8", "_f16"};
+        const std::string name = "eek_gemm_m64w" + std::to_string(t) + names[kind] + (sw ? "_swiglu" : "");
+        const Kernel* k = find_kernel(eng, name);
+        return launch(eng, name, cdiv(M, 64) * cdiv(N, small_cols(t, sw, kind == EE_GEMM_F8)), 1, k ? k->block : 64, g, stream);
+    }
     // The pipelined kernels stream whole 128-byte K stages; other K take the fallback.
     // Two pipelines: loader waves + MFMA waves (eek_gemm_*), and eight waves that
     // each load and compute (eek_gemm_*_w8).  Measured on MI355X (identical data,
@@ -799,6 +879,12 @@ EE_EXPORT int ee_gemm(ee_engine* eng, int32_t kind, const void* a, int64_t lda, 
                       int32_t* acc_out, ee_stream_t stream) {
     return gemm_impl(eng, kind, a, lda, b_nk, ldb, c, ldc, a_scale, b_scale, M, N, K, a_idx, c_idx, counts, tier,
                      acc_out, 0, stream);
+}
+
+EE_EXPORT int ee_gemm_small_waves(const ee_engine* eng, int32_t kind, int64_t M, int64_t N, int64_t K, int32_t swiglu) {
+    if (eng == nullptr || kind < EE_GEMM_I8 || kind > EE_GEMM_W8A16 || M <= 0 || N <= 0 || K <= 0) return 0;
+    const int64_t esz = kind == EE_GEMM_F16 ? 2 : 1;
+    return K * esz % 128 == 0 ? small_waves(eng, kind, M, N, K, swiglu != 0) : 0;
 }
 
 EE_EXPORT int ee_gemm_swiglu(ee_engine* eng, int32_t kind, const void* a, int64_t lda, const void* b_nk,
@@ -893,6 +979,15 @@ static int routed_impl(ee_engine* eng, const void* x, int64_t ld_x, int32_t M, i
                              ld_x, K, ldc, M, N, K, EE_TIER_FP16, sw};
         ra.mt_max = (int32_t)cdiv(M, 128) + 2;
         ra.f16_w8 = opt(eng, "gemm_variant") == 2;   // the FP16 pipeline ee_gemm picks (same f32 order)
+        bool dense = false;
+        if (const int t = small_routed_waves(eng, M, N, sw, dense)) {
+            ra.mt_max = (int32_t)cdiv(M, 64) + 2;
+            ra.t[2].b = b_i8;                            // the W8A16 kind: int8 codes and their scales
+            ra.t[2].b_scale = b_scale;
+            const std::string name = "eek_gemm_routed_m64w" + std::to_string(t) + (sw ? "_swiglu" : dense && t == 2 ? "_dense" : "");
+            const Kernel* k = find_kernel(eng, name);
+            return launch(eng, name, 24 + ra.mt_max * cdiv(N, small_cols(t, sw, false)), 1, k ? k->block : 64, ra, stream);
+        }
         const int64_t slots = (int64_t)ra.mt_max * cdiv(N, 128);
         // Large grids: the 256 x 256-tile routed kernel (same K order in every tier).
         // Its DMA addresses rows from the operands' starts with 32-bit offsets.
@@ -1254,12 +1349,18 @@ EE_EXPORT int ee_mlp_forward(ee_engine* eng, const void* x, int64_t ld_x, int64_
     const int tier = entropy < tau_low ? EE_TIER_INT8 : (entropy < tau_high ? EE_TIER_FP8 : EE_TIER_FP16);
     if (tier == EE_TIER_FP16) {
         const int sw = H % 64 == 0;                   // the pipelined W8A16 kernels: K * 2 % 128 == 0
-        if ((rc = gemm_impl(eng, EE_GEMM_F16, x, ld_x, gu_f16, H, sw ? (void*)w.act : (void*)w.gu, sw ? F : 2 * F,
-                            nullptr, nullptr, m, 2 * f, h, nullptr, nullptr, nullptr, 0, nullptr, sw, stream)))
+        // few rows: the small tiles from the int8 codes (the same bits from half the weight bytes)
+        const bool gu8 = aligned(gu_i8, 16) && aligned(gu_scale, 4) &&
+                         ee_gemm_small_waves(eng, EE_GEMM_W8A16, M, 2 * F, H, sw) > 0;
+        if ((rc = gemm_impl(eng, gu8 ? EE_GEMM_W8A16 : EE_GEMM_F16, x, ld_x, gu8 ? (const void*)gu_i8 : gu_f16, H,
+                            sw ? (void*)w.act : (void*)w.gu, sw ? F : 2 * F, nullptr, gu8 ? gu_scale : nullptr, m, 2 * f,
+                            h, nullptr, nullptr, nullptr, 0, nullptr, sw, stream)))
             return rc;
         if (!sw && (rc = silu_mul_impl(eng, w.gu, 2 * F, w.act, F, M, F, 1, stream))) return rc;
-        return ee_gemm(eng, EE_GEMM_F16, w.act, F, dn_f16, F, out, ldo, nullptr, nullptr, m, h, f, nullptr, nullptr,
-                       nullptr, 0, nullptr, stream);
+        const bool dn8 = aligned(dn_i8, 16) && aligned(dn_scale, 4) &&
+                         ee_gemm_small_waves(eng, EE_GEMM_W8A16, M, H, F, 0) > 0;
+        return ee_gemm(eng, dn8 ? EE_GEMM_W8A16 : EE_GEMM_F16, w.act, F, dn8 ? (const void*)dn_i8 : dn_f16, F, out, ldo,
+                       nullptr, dn8 ? dn_scale : nullptr, m, h, f, nullptr, nullptr, nullptr, 0, nullptr, stream);
     }
     const int32_t qmode = tier == EE_TIER_INT8 ? EE_QUANT_I8_DISPATCH : EE_QUANT_F8_ROW;
     const int32_t kind = tier == EE_TIER_INT8 ? EE_GEMM_I8 : EE_GEMM_F8;

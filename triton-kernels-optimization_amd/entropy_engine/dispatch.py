@@ -208,7 +208,7 @@ class EntropyDispatchedLinear(nn.Module):
             a, s = K.quantize_activations(x_2d, "fp8")
             out = K.gemm("fp8", a, pw.f8, s, pw.scale)
         else:
-            out = K.gemm("fp16", x_2d, pw.f16)
+            out = K.gemm_fp16_tier(x_2d, pw)
         if self.bias is not None:
             out = out + self.bias.unsqueeze(0)
         return out.reshape(orig_shape[:-1] + (self.out_features,))
@@ -501,7 +501,7 @@ class EntropyGatedLlama:
         else:
             pw = self.packed[key]
             if route is None:                # no entropy yet: FP16 tier (W8A16), as the reference's default
-                y = K.gemm("fp16", x2d, pw.f16, swiglu=swiglu)
+                y = K.gemm_fp16_tier(x2d, pw, swiglu=swiglu)
             else:
                 idx, counts = route
                 y = K.routed_linear(x2d, pw, idx, counts, swiglu=swiglu, quantized=quantized)

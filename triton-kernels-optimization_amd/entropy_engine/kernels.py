@@ -283,6 +283,18 @@ def gemm(kind: str, a: torch.Tensor, b_nk: torch.Tensor, a_scale=None, b_scale=N
     return c
 
 
+def gemm_fp16_tier(a: torch.Tensor, pw: PackedWeight, out=None, *, swiglu: bool = False) -> torch.Tensor:
+    """The FP16 (W8A16) tier of a packed weight: with few rows from the int8 codes, which the
+    small-GEMM kernels dequantise to pw.f16's values in registers (the same bits from half the
+    weight bytes), else from pw.f16."""
+    if a.shape[0] and pw.i8.data_ptr() % 16 == 0:
+        with torch.cuda.device(a.device):
+            small = _lib.lib().ee_gemm_small_waves(engine(), _lib.EE_GEMM_W8A16, a.shape[0], pw.N, pw.K, int(swiglu))
+        if small:
+            return gemm("w8a16", a, pw.i8, None, pw.scale, out=out, swiglu=swiglu)
+    return gemm("fp16", a, pw.f16, out=out, swiglu=swiglu)
+
+
 def _check_gemm_inputs(a, b_int8, b_scale):
     if a.dim() != 2 or b_int8.dim() != 2:
         raise ValueError("a must be [M, K] and b_int8 [K, N]")
@@ -316,7 +328,7 @@ def triton_fp16_gemm(a: torch.Tensor, b_int8: torch.Tensor, b_scale: torch.Tenso
     if not a.is_contiguous():
         a = a.contiguous()
     pw = prepare_weight(b_int8, b_scale)
-    return gemm("fp16", a, pw.f16)
+    return gemm_fp16_tier(a, pw)
 
 
 def fp8_tensor_gemm(a: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
