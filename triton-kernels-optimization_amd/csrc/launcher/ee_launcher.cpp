@@ -326,6 +326,7 @@ bool pick_se_cfg(int64_t len, int64_t rows, int64_t forced_wpr, int& vpt, int& w
 }
 
 int64_t opt(const ee_engine* e, const char* key) {
+    if (e->options.empty()) return 0;         // (only non-zero values are kept: the usual case, without a lookup)
     auto it = e->options.find(key);
     return it == e->options.end() ? 0 : it->second;
 }
@@ -494,7 +495,8 @@ EE_EXPORT int ee_engine_set_option(ee_engine* eng, const char* key, int64_t valu
     } else {
         return fail(EE_ERR_INVALID_ARG, "unknown option: " + k);
     }
-    eng->options[k] = value;
+    if (value) eng->options[k] = value;
+    else eng->options.erase(k);
     return EE_OK;
 }
 

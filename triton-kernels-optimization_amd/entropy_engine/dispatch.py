@@ -123,8 +123,8 @@ class RowEntropyRouter:
 
     def route(self, entropy: torch.Tensor):
         tier, idx, counts = K.route(entropy.contiguous().to(torch.float32), self.tau_low, self.tau_high)
-        c64 = counts.to(torch.int64)
-        self._totals = c64 if self._totals is None else self._totals + c64
+        # (int64 + int32 is one kernel, which widens counts as it adds)
+        self._totals = counts.to(torch.int64) if self._totals is None else self._totals + counts
         return tier, idx, counts
 
     def reset_stats(self):

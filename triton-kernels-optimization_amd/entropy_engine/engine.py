@@ -90,7 +90,7 @@ class CubinEngine:
                 raise RuntimeError(f"tensor on {t.device}, engine on {self.device}")
         b_nk = prepare_weight(b_int8, b_scale).i8
         out = torch.empty((M, N), dtype=torch.float16, device=self.device)
-        with torch.cuda.device(self.device):
+        with _lib.on_device(self.device):
             _lib.check(_lib.lib().ee_module_engine_forward(
                 self._handle, a_int8.data_ptr(), K, b_nk.data_ptr(), K, out.data_ptr(), N,
                 a_scale.data_ptr(), b_scale.data_ptr(), M, N, K, _lib.stream_handle()))
@@ -192,7 +192,7 @@ class EntropyMLPEngine:
         L = _lib.lib()
         nbytes = L.ee_mlp_workspace_bytes(M, self.H, self.F, int(h_rows is not None))
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=self.device)
-        with torch.cuda.device(self.device):
+        with _lib.on_device(self.device):
             _lib.check(L.ee_mlp_forward(
                 _lib.engine(), x.data_ptr(), self.H, M, self.H, self.F,
                 self.gu_i8.data_ptr(), self.gu_f8.data_ptr(), self.gu_f16.data_ptr(), self.gu_scale.data_ptr(),

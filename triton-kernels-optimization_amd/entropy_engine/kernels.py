@@ -24,7 +24,7 @@ import weakref
 import torch
 
 from . import _lib
-from ._lib import check, engine, ptr, stream_handle
+from ._lib import check, engine, engine_of, on_device, ptr, stream_handle, stream_of
 
 __all__ = [
     "triton_int8_gemm", "triton_fp8_gemm", "triton_fp16_gemm", "fused_softmax_entropy",
@@ -75,15 +75,15 @@ def softmax_entropy(x: torch.Tensor, causal: bool = False, probs: bool = True,
     p = None
     if probs:
         p = out_probs if out_probs is not None else torch.empty((R, S), dtype=torch.float16, device=dev)
-        if p.shape != (R, S) or p.dtype != torch.float16:
+        if out_probs is not None and (p.shape != (R, S) or p.dtype != torch.float16):
             raise ValueError("out_probs must be float16 of the logits' shape")
     ldp = _rowmajor(p, "probs") if p is not None else S
     h = torch.empty(R, dtype=torch.float32, device=dev)
     tier = torch.empty(R, dtype=torch.int32, device=dev) if thresholds is not None else None
     tl, th = thresholds if thresholds is not None else (0.0, 0.0)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_softmax_entropy(engine(), ptr(x), ptr(p), ptr(h), R, S, ldx, ldp, int(bool(causal)),
-                                            ptr(tier), float(tl), float(th), stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_softmax_entropy(engine_of(dev), ptr(x), ptr(p), ptr(h), R, S, ldx, ldp, int(bool(causal)),
+                                            ptr(tier), float(tl), float(th), stream_of(dev)))
     return p, h, tier
 
 
@@ -123,9 +123,9 @@ def quantize_activations(a: torch.Tensor, mode: str = "dispatcher", idx=None, co
     code_dtype = torch.uint8 if mode == "fp8" else torch.int8
     codes = out_codes if out_codes is not None else torch.empty((M, K), dtype=code_dtype, device=dev)
     scale = out_scale if out_scale is not None else torch.empty(M, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_quant_act(engine(), ptr(a), M, K, lda, _MODES[mode], ptr(codes), _rowmajor(codes, "codes"),
-                                      ptr(scale), ptr(idx), ptr(counts), int(tier), stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_quant_act(engine_of(dev), ptr(a), M, K, lda, _MODES[mode], ptr(codes), _rowmajor(codes, "codes"),
+                                      ptr(scale), ptr(idx), ptr(counts), int(tier), stream_of(dev)))
     return codes, scale
 
 
@@ -144,9 +144,9 @@ def quantize_tensor_fp8(x: torch.Tensor):
     codes = torch.empty((R, K), dtype=torch.uint8, device=dev)
     scale = torch.empty(R, dtype=torch.float32, device=dev)
     ws = torch.empty(_lib.EE_TENSOR_WS_FLOATS, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_quant_tensor_f8(engine(), ptr(x), R, K, ldx, ptr(codes), K, ptr(scale), ptr(ws),
-                                            stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_quant_tensor_f8(engine_of(dev), ptr(x), R, K, ldx, ptr(codes), K, ptr(scale), ptr(ws),
+                                            stream_of(dev)))
     return codes, scale
 
 
@@ -161,8 +161,8 @@ def quantize_weight_codes(weight: torch.Tensor):
     N, K = w.shape
     codes = torch.empty((N, K), dtype=torch.int8, device=dev)
     scale = torch.empty(N, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_quant_weight_i8(engine(), ptr(w), N, K, K, ptr(codes), K, ptr(scale), stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_quant_weight_i8(engine_of(dev), ptr(w), N, K, K, ptr(codes), K, ptr(scale), stream_of(dev)))
     return codes, scale
 
 
@@ -172,8 +172,8 @@ def transpose_i8(src: torch.Tensor) -> torch.Tensor:
         raise TypeError("transpose_i8 takes int8/uint8")
     R, C = src.shape
     dst = torch.empty((C, R), dtype=src.dtype, device=dev)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_transpose_i8(engine(), ptr(src), R, C, _rowmajor(src, "src"), ptr(dst), R, stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_transpose_i8(engine_of(dev), ptr(src), R, C, _rowmajor(src, "src"), ptr(dst), R, stream_of(dev)))
     return dst
 
 
@@ -206,7 +206,7 @@ class PackedWeight:
         if self._f8 is None:
             N, K = self.i8.shape
             out = torch.empty((N, K), dtype=torch.uint8, device=self.i8.device)
-            with torch.cuda.device(self.i8.device):
+            with on_device(self.i8.device):
                 check(_lib.lib().ee_pack_b_f8(engine(), ptr(self.i8), N, K, K, ptr(out), K, stream_handle()))
             self._f8 = out
         return self._f8
@@ -216,7 +216,7 @@ class PackedWeight:
         if self._f16 is None:
             N, K = self.i8.shape
             out = torch.empty((N, K), dtype=torch.float16, device=self.i8.device)
-            with torch.cuda.device(self.i8.device):
+            with on_device(self.i8.device):
                 check(_lib.lib().ee_pack_b_f16(engine(), ptr(self.i8), ptr(self.scale), N, K, K, ptr(out), K,
                                                stream_handle()))
             self._f16 = out
@@ -269,17 +269,17 @@ def gemm(kind: str, a: torch.Tensor, b_nk: torch.Tensor, a_scale=None, b_scale=N
     if a.shape[1] != K:
         raise ValueError(f"K mismatch: a is {tuple(a.shape)}, b is [{N}, {K}] in operand order")
     c = out if out is not None else torch.empty((M, N // 2 if swiglu else N), dtype=torch.float16, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         if swiglu:
             if acc_out is not None:
                 raise ValueError("acc_out is not available with swiglu")
-            check(_lib.lib().ee_gemm_swiglu(engine(), _KINDS[kind], ptr(a), lda, ptr(b_nk), ldb, ptr(c),
+            check(_lib.lib().ee_gemm_swiglu(engine_of(dev), _KINDS[kind], ptr(a), lda, ptr(b_nk), ldb, ptr(c),
                                             _rowmajor(c, "act"), ptr(a_scale), ptr(b_scale), M, N, K, ptr(a_idx),
-                                            ptr(c_idx), ptr(counts), int(tier), stream_handle()))
+                                            ptr(c_idx), ptr(counts), int(tier), stream_of(dev)))
         else:
-            check(_lib.lib().ee_gemm(engine(), _KINDS[kind], ptr(a), lda, ptr(b_nk), ldb, ptr(c), _rowmajor(c, "c"),
+            check(_lib.lib().ee_gemm(engine_of(dev), _KINDS[kind], ptr(a), lda, ptr(b_nk), ldb, ptr(c), _rowmajor(c, "c"),
                                      ptr(a_scale), ptr(b_scale), M, N, K, ptr(a_idx), ptr(c_idx), ptr(counts),
-                                     int(tier), ptr(acc_out), stream_handle()))
+                                     int(tier), ptr(acc_out), stream_of(dev)))
     return c
 
 
@@ -287,10 +287,8 @@ def gemm_fp16_tier(a: torch.Tensor, pw: PackedWeight, out=None, *, swiglu: bool 
     """The FP16 (W8A16) tier of a packed weight: with few rows from the int8 codes, which the
     small-GEMM kernels dequantise to pw.f16's values in registers (the same bits from half the
     weight bytes), else from pw.f16."""
-    if a.shape[0] and pw.i8.data_ptr() % 16 == 0:
-        with torch.cuda.device(a.device):
-            small = _lib.lib().ee_gemm_small_waves(engine(), _lib.EE_GEMM_W8A16, a.shape[0], pw.N, pw.K, int(swiglu))
-        if small:
+    if a.is_cuda and a.shape[0] and pw.i8.data_ptr() % 16 == 0:
+        if _lib.lib().ee_gemm_small_waves(engine_of(a.device), _lib.EE_GEMM_W8A16, a.shape[0], pw.N, pw.K, int(swiglu)):
             return gemm("w8a16", a, pw.i8, None, pw.scale, out=out, swiglu=swiglu)
     return gemm("fp16", a, pw.f16, out=out, swiglu=swiglu)
 
@@ -350,9 +348,9 @@ def route(h: torch.Tensor, tau_low: float, tau_high: float):
     tier = torch.empty(R, dtype=torch.int32, device=dev)
     idx = torch.empty(R, dtype=torch.int32, device=dev)
     counts = torch.empty(3, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_route(engine(), ptr(h), R, float(tau_low), float(tau_high), ptr(tier), ptr(idx),
-                                  ptr(counts), stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_route(engine_of(dev), ptr(h), R, float(tau_low), float(tau_high), ptr(tier), ptr(idx),
+                                  ptr(counts), stream_of(dev)))
     return tier, idx, counts
 
 
@@ -368,9 +366,9 @@ def route_heads(h: torch.Tensor, tau_low: float, tau_high: float):
     tier = torch.empty(R, dtype=torch.int32, device=dev)
     idx = torch.empty(R, dtype=torch.int32, device=dev)
     counts = torch.empty(3, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_route_heads(engine(), ptr(h), B, Hh, S, float(tau_low), float(tau_high), ptr(tier),
-                                        ptr(idx), ptr(counts), stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_route_heads(engine_of(dev), ptr(h), B, Hh, S, float(tau_low), float(tau_high), ptr(tier),
+                                        ptr(idx), ptr(counts), stream_of(dev)))
     return tier, idx, counts
 
 
@@ -384,10 +382,10 @@ def row_copy(src: torch.Tensor, idx: torch.Tensor, counts=None, tier: int = 0, s
     if out is None:
         out = torch.empty((rows, src.shape[1]) if not scatter else src.shape, dtype=src.dtype, device=dev)
     es = src.element_size()
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_row_copy(engine(), ptr(src), _rowmajor(src, "src") * es, ptr(out),
+    with on_device(dev):
+        check(_lib.lib().ee_row_copy(engine_of(dev), ptr(src), _rowmajor(src, "src") * es, ptr(out),
                                      _rowmajor(out, "out") * es, rows, src.shape[1] * es, ptr(idx), ptr(counts),
-                                     int(tier), int(bool(scatter)), stream_handle()))
+                                     int(tier), int(bool(scatter)), stream_of(dev)))
     return out
 
 
@@ -419,10 +417,10 @@ def routed_linear(x: torch.Tensor, pw: PackedWeight, idx: torch.Tensor, counts: 
                          torch.empty(M, dtype=torch.float32, device=dev))
         ws_codes, ws_scale = workspace
         fn = _lib.lib().ee_routed_linear_swiglu if swiglu else _lib.lib().ee_routed_linear
-    with torch.cuda.device(dev):
-        check(fn(engine(), ptr(x), _rowmajor(x, "x"), M, K, N, ptr(idx), ptr(counts), ptr(pw.i8), ptr(pw.f8),
+    with on_device(dev):
+        check(fn(engine_of(dev), ptr(x), _rowmajor(x, "x"), M, K, N, ptr(idx), ptr(counts), ptr(pw.i8), ptr(pw.f8),
                  ptr(pw.f16), ptr(pw.scale), ptr(c), _rowmajor(c, "out"), ptr(ws_codes), ptr(ws_scale),
-                 stream_handle()))
+                 stream_of(dev)))
     return c
 
 
@@ -435,9 +433,9 @@ def interleave_gate_up(t: torch.Tensor) -> torch.Tensor:
         raise ValueError("gate|up needs 2F rows with F % 32 == 0")
     rb = t[0].numel() * t.element_size() if t.dim() > 1 else t.element_size()
     out = torch.empty_like(t)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_interleave_gate_up(engine(), ptr(t), rb, ptr(out), rb, t.shape[0] // 2, rb,
-                                               stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_interleave_gate_up(engine_of(dev), ptr(t), rb, ptr(out), rb, t.shape[0] // 2, rb,
+                                               stream_of(dev)))
     return out
 
 
@@ -455,9 +453,9 @@ def silu_mul(gu: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         raise ValueError("gu must hold [gate | up]: an even number of columns")
     F = F2 // 2
     act = out if out is not None else torch.empty((M, F), dtype=torch.float16, device=dev)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_silu_mul(engine(), ptr(gu), _rowmajor(gu, "gu"), ptr(act), _rowmajor(act, "out"), M, F,
-                                     stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_silu_mul(engine_of(dev), ptr(gu), _rowmajor(gu, "gu"), ptr(act), _rowmajor(act, "out"), M, F,
+                                     stream_of(dev)))
     return act
 
 
@@ -484,11 +482,11 @@ def add_rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, y: torch.Tensor | 
     each op in torch's precision; rows of the last dimension D (D % 8 == 0, D <= 4096)."""
     dev = _require_cuda(x, w, y)
     x2, y2, s, n, w, T, D = _rmsnorm_operands(x, w, y)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_add_rmsnorm(engine(), ptr(x2), _rowmajor(x2, "x"), ptr(y2),
+    with on_device(dev):
+        check(_lib.lib().ee_add_rmsnorm(engine_of(dev), ptr(x2), _rowmajor(x2, "x"), ptr(y2),
                                         _rowmajor(y2, "y") if y2 is not None else D, ptr(w),
                                         ptr(s) if y is not None else None, D, ptr(n), D, T, D, float(eps),
-                                        stream_handle()))
+                                        stream_of(dev)))
     return s.view(x.shape), n.view(x.shape)
 
 
@@ -514,11 +512,11 @@ def add_rmsnorm_route(x: torch.Tensor, w: torch.Tensor, eps: float, y: torch.Ten
         n = n_out
     codes = torch.empty((T, D), dtype=torch.uint8, device=dev)
     scale = torch.empty(T, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_add_rmsnorm_route(engine(), ptr(x2), _rowmajor(x2, "x"), ptr(y2),
+    with on_device(dev):
+        check(_lib.lib().ee_add_rmsnorm_route(engine_of(dev), ptr(x2), _rowmajor(x2, "x"), ptr(y2),
                                               _rowmajor(y2, "y") if y2 is not None else D, ptr(w),
                                               ptr(s) if y is not None else None, D, ptr(n), D, T, D, float(eps),
-                                              ptr(idx), ptr(counts), ptr(codes), D, ptr(scale), stream_handle()))
+                                              ptr(idx), ptr(counts), ptr(codes), D, ptr(scale), stream_of(dev)))
     return s.view(x.shape), (n.view(x.shape) if n_out is not None else None), codes, scale
 
 
@@ -536,9 +534,9 @@ def qkv_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, B: int, S:
     k = torch.empty((B, Hkv, S, d), dtype=torch.float16, device=dev)
     v = torch.empty((B, Hkv, d, S) if v_transposed else (B, Hkv, S, d), dtype=torch.float16, device=dev)
     fn = _lib.lib().ee_qkv_rope_vt if v_transposed else _lib.lib().ee_qkv_rope
-    with torch.cuda.device(dev):
-        check(fn(engine(), ptr(qkv), ld, ptr(cos), ptr(sin), ptr(q), ptr(k), ptr(v), B, S, Hq, Hkv, d, float(q_scale),
-                 stream_handle()))
+    with on_device(dev):
+        check(fn(engine_of(dev), ptr(qkv), ld, ptr(cos), ptr(sin), ptr(q), ptr(k), ptr(v), B, S, Hq, Hkv, d, float(q_scale),
+                 stream_of(dev)))
     return q, k, v
 
 
@@ -563,7 +561,7 @@ def attention_causal(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, out: to
         out = torch.empty((B * S, Hq * d), dtype=torch.float16, device=dev)
     ld_out = _rowmajor(out, "out")
     h = torch.empty((B, Hq, S), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        check(_lib.lib().ee_attention_causal(engine(), ptr(q), ptr(k), ptr(vt), ptr(out), ld_out, ptr(h), B, S, Hq,
-                                             Hkv, d, stream_handle()))
+    with on_device(dev):
+        check(_lib.lib().ee_attention_causal(engine_of(dev), ptr(q), ptr(k), ptr(vt), ptr(out), ld_out, ptr(h), B, S, Hq,
+                                             Hkv, d, stream_of(dev)))
     return out, h
