@@ -16,6 +16,10 @@
 // once: 2 bytes in + 2 bytes out per element + 4 bytes of H per row.
 #include "../common/ee_device.h"
 
+// 16 bytes of a row, which starts at any multiple of 2 bytes: gfx950 loads and stores them at any
+// address (the compiler emits the same global_load_dwordx4 for either alignment).
+typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
+
 #define LOG2E 1.4426950408889634f
 #define LN2 0.69314718055994531f
 
@@ -83,6 +87,16 @@ EE_DEV uint32_t scale_pack_f16x2(float e0, float e1, float s) {
     return r;
 }
 
+// A row whose max is within 104 of the lowest fp16 value: -inf entries (masked or padding) clamped to
+// -65504 would count beside it (e^-104 is the first e that is 0 in f32), so the row is moved up by 32768
+// first, exactly (its finite entries are multiples of 32 from -65504 up; -inf stays).
+#define NEAR_LOWEST(m) ((m) < -65376.0f)
+#define LOW_SHIFT 32768.0f
+EE_DEV uint32_t shift_up(uint32_t u) {
+    const f16x2 s = {(f16)LOW_SHIFT, (f16)LOW_SHIFT};
+    return bits_of(f16x2_from_bits(u) + s);
+}
+
 // Row kernel: WPR wave64s per row (one to eight), VPT 16-byte vectors per lane
 // (S <= VPT * WPR * 512).  Passes over the registers:
 //  1. max with packed fp16 IEEE maximum (NaN anywhere, or no finite entry,
@@ -109,8 +123,8 @@ EE_DEV void se_load(const EeSoftmaxArgs& a, int64_t r, int wr, int lane, u32x4 (
     for (int j = 0; j < VPT; ++j) {
         const int c0 = ((j * WPR + wr) * 64 + lane) * 8;
         if (c0 + 8 <= nvalid) {
-            if constexpr (NT) v[j] = __builtin_nontemporal_load((const u32x4*)(xr + c0));
-            else v[j] = *(const u32x4*)(xr + c0);
+            if constexpr (NT) v[j] = __builtin_nontemporal_load((const u32x4_u*)(xr + c0));
+            else v[j] = *(const u32x4_u*)(xr + c0);
         } else {
             uint16_t e[8];
 #pragma unroll
@@ -156,6 +170,13 @@ EE_DEV void se_process(const EeSoftmaxArgs& a, u32x4 (&v)[VPT], int64_t row, boo
     const bool dead = !(m > -INFINITY);
     const bool has_max = __builtin_amdgcn_ballot_w64(m_lane == m) != 0;   // wave-uniform
     if (dead) m = 0.0f;
+    if (NEAR_LOWEST(m)) {                             // (wave-uniform)
+#pragma unroll
+        for (int j = 0; j < VPT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[j][i] = shift_up(v[j][i]);
+        m += LOW_SHIFT;
+    }
     const float negm = -m;
 
     // ---- 2. -inf -> -65504 (after the max, so NaN rows stay dead).  IEEE maximum
@@ -244,7 +265,7 @@ EE_DEV void se_process(const EeSoftmaxArgs& a, u32x4 (&v)[VPT], int64_t row, boo
             if (c0 + 8 <= S) {
                 // written once, read by a later kernel: non-temporal (measured 5% faster
                 // at [4096, 14336], where the kernel runs at ~93% of a plain copy)
-                __builtin_nontemporal_store(o, (u32x4*)(pr + c0));
+                __builtin_nontemporal_store(o, (u32x4_u*)(pr + c0));
             } else {
     #pragma unroll
                 for (int i = 0; i < 8; ++i)
@@ -289,9 +310,162 @@ EE_DEV void softmax_entropy_rows(const EeSoftmaxArgs& a) {
     }
 }
 
+// Rows of up to 1024 columns in groups of LPR lanes (16 or 32): a wave works on 64 / LPR
+// consecutive rows at once, each lane holding VPT vectors of its row (S <= 8 LPR VPT).
+// With one wave per row the kernel is bound by its instructions there, not by memory: per row the
+// wave reductions (max, Z', T, c0: ~130 instructions) cost as much as the row's 8 elements per
+// lane.  Here they serve 4 (2) rows, over 16 lanes by DPP alone.  Vectors past every row's
+// causal limit are neither loaded nor evaluated.  Measured at [131072, 512] with
+// probabilities: causal 59.9 -> 35.4 us (5.7 TB/s of the bytes the rows cannot do
+// without), all columns 54.0 -> 42.4 us (6.3 TB/s, a large copy's rate).
+// Same steps, per-element arithmetic and results as se_process (the sums in another order).
+template <int LPR>
+EE_DEV float grp_max(float v) {                    // IEEE maximum over the lane's group
+    v = fmaximum(v, dpp_f32<0xB1>(v));
+    v = fmaximum(v, dpp_f32<0x4E>(v));
+    v = fmaximum(v, dpp_f32<0x141>(v));
+    v = fmaximum(v, dpp_f32<0x140>(v));
+    if constexpr (LPR == 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaximum(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    return v;
+}
+template <int LPR>
+EE_DEV float grp_sum(float v) {
+    v += dpp_f32<0xB1>(v);
+    v += dpp_f32<0x4E>(v);
+    v += dpp_f32<0x141>(v);
+    v += dpp_f32<0x140>(v);
+    if constexpr (LPR == 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    return v;
+}
+
+template <int VPT, int LPR>
+EE_DEV void softmax_entropy_group(const EeSoftmaxArgs& a) {
+    constexpr int RPW = 64 / LPR;
+    const int lane = lane_id(), gl = lane & (LPR - 1), grp = lane / LPR;
+    const int S = a.S;
+    // (the launcher keeps rows below 2^31 and S >= 16)
+    const uint32_t row0 = __builtin_amdgcn_readfirstlane((blockIdx.x * (EE_BLOCK / 64) + wave_id()) * RPW);
+    if (row0 >= (uint32_t)a.rows) return;
+    const uint32_t row = min(row0 + grp, (uint32_t)a.rows - 1);   // past the end: the last row again, not stored
+    int nvalid = S, nmax = S;                      // columns of the row, and of the wave's longest row
+    if (a.causal) {
+        const int p0 = __builtin_amdgcn_readfirstlane((int)(row0 % (uint32_t)S));
+        const int p = p0 + (int)(row - row0);
+        nvalid = (p >= S ? p - S : p) + 1;
+        nmax = min(S, p0 + RPW);                   // (a wave that wraps holds row S - 1)
+    }
+    const uint16_t* xr = a.x + (int64_t)row * a.ld_x;
+    u32x4 v[VPT];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        v[j] = u32x4{0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u};
+        if (j * LPR * 8 < nmax) {                  // uniform
+            const int c0 = (j * LPR + gl) * 8;
+            if (c0 < nvalid) {
+                if (c0 + 8 <= S) {
+                    v[j] = *(const u32x4_u*)(xr + c0);
+                } else {                           // the row's last, partial vector
+                    uint16_t e[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) e[i] = c0 + i < S ? xr[c0 + i] : (uint16_t)0xFC00u;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[j][i] = e[2 * i] | ((uint32_t)e[2 * i + 1] << 16);
+                }
+            }
+        }
+    }
+    if (a.causal) {                                // -inf past the limit, in the vector that it cuts
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            const int k = nvalid - (j * LPR + gl) * 8;
+            if (j * LPR * 8 < nmax && k > 0 && k < 8) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (k < 2 * i + 2) v[j][i] = k == 2 * i + 1 ? (v[j][i] & 0xffffu) | 0xFC000000u : 0xFC00FC00u;
+                }
+            }
+        }
+    }
+    f16x2 mx2 = f16x2_from_bits(0xFC00FC00u);
+#pragma unroll
+    for (int j = 0; j < VPT; ++j)
+        if (j * LPR * 8 < nmax) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mx2 = __builtin_elementwise_maximum(mx2, f16x2_from_bits(v[j][i]));
+        }
+    float m = grp_max<LPR>(fmaximum((float)mx2.x, (float)mx2.y));
+    const bool dead = !(m > -INFINITY);
+    if (dead) m = 0.0f;
+    if (__builtin_amdgcn_ballot_w64(NEAR_LOWEST(m)) != 0) {
+        if (NEAR_LOWEST(m)) {
+#pragma unroll
+            for (int j = 0; j < VPT; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[j][i] = shift_up(v[j][i]);
+            m += LOW_SHIFT;
+        }
+    }
+    const float negm = -m;
+    const f16x2 lowest = f16x2_from_bits(0xFBFFFBFFu);
+    float ek[VPT * 8];
+    float z0 = 0.f, z1 = 0.f, t0 = 0.f, t1 = 0.f;
+    int cnt = 0;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        if (j * LPR * 8 < nmax) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t u = bits_of(__builtin_elementwise_maximum(f16x2_from_bits(v[j][i >> 1]), lowest));
+                const float s = (i & 1) ? sub_hi(u, negm) : sub_lo(u, negm);
+                const float e = __builtin_amdgcn_exp2f(s * LOG2E);
+                const bool at_max = s == 0.0f;
+                cnt += at_max ? 1 : 0;
+                if (i & 1) { z1 += at_max ? 0.0f : e; t1 = fmaf(e, s, t1); }
+                else       { z0 += at_max ? 0.0f : e; t0 = fmaf(e, s, t0); }
+                ek[j * 8 + i] = e;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ek[j * 8 + i] = 0.0f;
+        }
+    }
+    const float z = grp_sum<LPR>(z0 + z1), t = grp_sum<LPR>(t0 + t1), cz = grp_sum<LPR>((float)cnt);
+    const bool mine = row0 + grp < (uint32_t)a.rows;
+    if (a.p != nullptr && mine) {
+        const float invZ = dead ? NAN : __builtin_amdgcn_rcpf(cz + z);
+        uint16_t* pr = a.p + (int64_t)row * a.ld_p;
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            const int c0 = (j * LPR + gl) * 8;
+            if (c0 >= S) continue;
+            const float* ev = ek + j * 8;
+            const u32x4 o{scale_pack_f16x2(ev[0], ev[1], invZ), scale_pack_f16x2(ev[2], ev[3], invZ),
+                          scale_pack_f16x2(ev[4], ev[5], invZ), scale_pack_f16x2(ev[6], ev[7], invZ)};
+            if (c0 + 8 <= S) {
+                __builtin_nontemporal_store(o, (u32x4_u*)(pr + c0));
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (c0 + i < S) pr[c0 + i] = (uint16_t)(o[i >> 1] >> ((i & 1) * 16));
+            }
+        }
+    }
+    const float H = dead ? NAN : entropy_from(cz, z, t);
+    if (gl == 0 && mine) {
+        a.h[row] = H;
+        if (a.tier) a.tier[row] = tier_of(H, a.tau_low, a.tau_high);
+    }
+}
+
 // Any row length, any alignment: one wave per row, three passes over the row
-// (max, sums, store) with 2-byte loads.  Used when the vector kernel's
-// preconditions (16-byte aligned rows, S <= 8 * 512 * 4) do not hold.
+// (max, sums, store) with 2-byte loads.  Used for rows that the vector kernels do not
+// hold (S > 8 * 8 * 512).
 EE_DEV void softmax_entropy_generic(const EeSoftmaxArgs& a) {
     const int lane = lane_id();
     const int64_t row = (int64_t)blockIdx.x * 4 + wave_id();
@@ -375,6 +549,16 @@ EE_SE_VEC_8W(4, 8)
 EE_SE_ROWS(1, 2)
 EE_SE_ROWS(1, 4)
 EE_SE_ROWS(2, 2)
+#define EE_SE_GROUP(V, L) \
+    extern "C" __global__ void __launch_bounds__(EE_BLOCK) eek_softmax_entropy_g##L##_v##V(EeSoftmaxArgs a) { \
+        softmax_entropy_group<V, L>(a);                                                                 \
+    }
+EE_SE_GROUP(1, 16)
+EE_SE_GROUP(2, 16)
+EE_SE_GROUP(3, 16)
+EE_SE_GROUP(4, 16)
+EE_SE_GROUP(3, 32)
+EE_SE_GROUP(4, 32)
 // rows longer than 4 * 8 * 512: eight waves, probabilities from recomputed e
 EE_SE_VEC(5, 8)
 EE_SE_VEC(6, 8)

@@ -468,6 +468,8 @@ EE_EXPORT int ee_engine_set_option(ee_engine* eng, const char* key, int64_t valu
         if (value < 0 || value > 8) return fail(EE_ERR_INVALID_ARG, k + " must be 0 (auto) or 1..8");
     } else if (k == "se_nt") {
         if (value < 0 || value > 2) return fail(EE_ERR_INVALID_ARG, k + " must be 0 (auto), 1 (off) or 2 (on)");
+    } else if (k == "se_group") {
+        if (value < 0 || value > 2) return fail(EE_ERR_INVALID_ARG, k + " must be 0 (auto), 1 (off) or 2 (on)");
     } else if (k == "se_rpw") {
         if (value != 0 && value != 1 && value != 2 && value != 4)
             return fail(EE_ERR_INVALID_ARG, k + " must be 0 (auto), 1, 2 or 4");
@@ -525,9 +527,22 @@ EE_EXPORT int ee_softmax_entropy(ee_engine* eng, const void* x, void* p, float* 
     const int64_t nt_opt = opt(eng, "se_nt");
     const int64_t se_bytes = rows * S * 2 * (p != nullptr ? 2 : 1);
     const bool nt = nt_opt == 2 || (nt_opt == 0 && se_bytes > (int64_t(256) << 20));
-    const bool vec_ok = aligned(x, 16) && aligned(p, 16) && ld_x % 8 == 0 && (p == nullptr || ld_p % 8 == 0);
+    // Rows of 16 to 1024 columns: 4 or 2 rows per wave (eek_softmax_entropy_g*), where the rows then still
+    // fill the chip.  Measured, us, one row (or two in turn) per wave against this: [131072, 512] causal 59.9 /
+    // 35.4, all columns 54.0 / 42.4; [40000, 301] 21.6 / 11.7; [16384, 128] 8.6 / 4.1; [4096, 512] 4.3 / 4.15 but
+    // [2048, 512] 3.5 / 4.0, [64, 384] 3.2 / 3.4; two rows per wave: [2048, 1024] causal 4.5 / 4.4, [8192, 768] 8.3 /
+    // 7.3, [16384, 1000] 13.1 / 12.7 but [8192, 1000] 8.5 / 9.0, [512, 777] 4.0 / 4.6.
+    // Option "se_group": 0 auto, 1 off, 2 wherever the kernel takes the shape.
+    const int64_t g_opt = opt(eng, "se_group");
+    const bool g_ok = S >= 16 && S <= 1024 && rows < (int64_t(1) << 31);
+    const bool g_fill = S <= 384 || rows >= (S <= 512 ? 4096 : S <= 768 || causal ? 2048 : 16384);
+    if (g_ok && (g_opt == 2 || (g_opt == 0 && g_fill && !opt(eng, "se_wpr") && !opt(eng, "se_rpw")))) {
+        const int lpr = S <= 512 ? 16 : 32;
+        const std::string name = "eek_softmax_entropy_g" + std::to_string(lpr) + "_v" + std::to_string(cdiv(S, 8 * lpr));
+        return launch(eng, name, cdiv(rows, 4 * (64 / lpr)), 1, EE_BLOCK, a, stream);
+    }
     int vpt = 0, wpr = 0;
-    if (vec_ok && pick_se_cfg(S, rows, opt(eng, "se_wpr"), vpt, wpr)) {
+    if (pick_se_cfg(S, rows, opt(eng, "se_wpr"), vpt, wpr)) {
         // Short single-wave rows: several rows per wave (their loads issued together)
         // once there are rows enough to keep every CU busy.  Option "se_rpw": 1 = one
         // row per wave, 2 or 4 = that many where the variant exists.
