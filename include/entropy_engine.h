@@ -201,6 +201,10 @@ int ee_route(ee_engine* eng, const float* h, int64_t rows, double tau_low, doubl
 int ee_route_heads(ee_engine* eng, const float* h, int32_t B, int32_t heads, int32_t S, double tau_low,
                    double tau_high, int32_t* tier, int32_t* idx, int32_t* counts, ee_stream_t stream);
 
+/* out[r] = mean of x[r, 0 .. n-1] (f32, x [rows, n] contiguous): the mean row entropy per
+ * batch element of EE/python/kernels.py:452. */
+int ee_row_mean(ee_engine* eng, const float* x, int64_t rows, int32_t n, float* out, ee_stream_t stream);
+
 /* Row gather (scatter = 0: dst[r] = src[idx[off+r]]) or scatter
  * (scatter = 1: dst[idx[off+r]] = src[r]) for r < counts[tier] (or rows). */
 int ee_row_copy(ee_engine* eng, const void* src, int64_t ld_src_bytes, void* dst, int64_t ld_dst_bytes,

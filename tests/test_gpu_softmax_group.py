@@ -1,5 +1,5 @@
 """Several rows per wave (eek_softmax_entropy_g*), rows at any 2-byte alignment in the vector
-kernels, against the oracle."""
+kernels, and the row mean, against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -121,3 +121,14 @@ def test_softmax_unaligned_long_rows(ee, orc, R, S, causal):
     check_probs(host(p), P_ref)
     assert torch.isnan(out[5:].view(R, S + 2)[:, S:]).all()
 
+
+@pytest.mark.parametrize("B,H,S", [(1, 1, 1), (3, 5, 33), (2, 7, 64), (8, 32, 512), (2, 3, 171)])
+def test_row_mean(ee, B, H, S):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(S)
+    x = torch.randn(B, H, S, S, generator=g, device="cuda").half()
+    _, ent = ee.fused_softmax_entropy(x, causal=True)
+    _, h, _ = ee.softmax_entropy(x.view(B * H * S, S), causal=True)
+    ref = h.double().view(B, -1).mean(dim=1)
+    # f32 sums of n non-negative values, at most 64 of them in a row
+    assert ((ent.double() - ref).abs() <= 64 * 2.0 ** -23 * ref + 1e-30).all()

@@ -99,7 +99,7 @@ struct EeRoutedGemmArgs {
 struct EeRouteArgs {
     const float* h;         // [rows], or with heads > 1 [rows / seq, heads, seq]: row r = b * seq + s
                             // routes on the mean over heads of h[b, :, s]
-    int32_t* tier;          // [rows]
+    int32_t* tier;          // [rows] (eek_route_mean: [rows] f32 means)
     int32_t* idx;           // [rows]: rows of tier 0, then tier 1, then tier 2
     int32_t* counts;        // [3]
     int64_t rows;

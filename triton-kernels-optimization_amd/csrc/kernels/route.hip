@@ -115,6 +115,38 @@ EE_DEV void route_chunk1(const EeRouteArgs& a, int32_t (*wsum)[3], int tid, int 
     route_place(a, r0, t, pos);
 }
 
+// Means of f32 rows (the dispatcher's mean row entropy per batch element): row b of h [rows, seq],
+// one 1024-thread workgroup each, to the b-th f32 of `tier`.  Latency-bound: 8 rows of 16384 2.6 us
+// (torch's reduction 4.9), of 65536 3.9 (7.6); one row of 262144 10.7 (9.6: more workgroups pay there).
+extern "C" __global__ void __launch_bounds__(1024) eek_route_mean(EeRouteArgs a) {
+    __shared__ float part[16];
+    const int n = a.seq, tid = (int)threadIdx.x;
+    const float* x = a.h + (int64_t)blockIdx.x * n;
+    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
+    if (((uintptr_t)x & 15) == 0) {
+        const int q = n >> 2;
+        for (int i = tid; i < q; i += 1024) {
+            const f32x4 v = ((const f32x4*)x)[i];
+            s0 += v[0];
+            s1 += v[1];
+            s2 += v[2];
+            s3 += v[3];
+        }
+        if (tid < (n & 3)) s0 += x[4 * q + tid];
+    } else {
+        for (int i = tid; i < n; i += 1024) s0 += x[i];
+    }
+    const float w = wave_sum((s0 + s1) + (s2 + s3));
+    if (lane_id() == 0) part[wave_id()] = w;
+    __syncthreads();
+    if (tid == 0) {
+        float t = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) t += part[i];
+        ((float*)a.tier)[blockIdx.x] = t / (float)n;
+    }
+}
+
 extern "C" __global__ void __launch_bounds__(1024) eek_route(EeRouteArgs a) {
     __shared__ int32_t wsum[16][3];
     __shared__ int32_t base[3];

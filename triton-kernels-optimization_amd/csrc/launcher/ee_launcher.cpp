@@ -942,6 +942,15 @@ EE_EXPORT int ee_route_heads(ee_engine* eng, const float* h, int32_t B, int32_t 
     return launch(eng, "eek_route", 1, 1, 1024, a, stream);
 }
 
+EE_EXPORT int ee_row_mean(ee_engine* eng, const float* x, int64_t rows, int32_t n, float* out, ee_stream_t stream) {
+    if (eng == nullptr || x == nullptr || out == nullptr) return fail(EE_ERR_INVALID_ARG, "NULL argument");
+    if (rows < 0 || n <= 0) return fail(EE_ERR_INVALID_ARG, "need rows >= 0 and n > 0");
+    if (!aligned(x, 4) || !aligned(out, 4)) return fail(EE_ERR_INVALID_ARG, "misaligned pointer");
+    if (rows == 0) return EE_OK;
+    EeRouteArgs a{x, (int32_t*)out, nullptr, nullptr, rows, 0.0, 0.0, 1, n};
+    return launch(eng, "eek_route_mean", rows, 1, 1024, a, stream);
+}
+
 EE_EXPORT int ee_row_copy(ee_engine* eng, const void* src, int64_t ld_src_bytes, void* dst, int64_t ld_dst_bytes,
                           int64_t rows, int64_t row_bytes, const int32_t* idx, const int32_t* counts, int32_t tier,
                           int32_t scatter, ee_stream_t stream) {

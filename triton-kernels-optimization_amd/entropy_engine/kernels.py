@@ -97,7 +97,13 @@ def fused_softmax_entropy(logits: torch.Tensor, causal: bool = True) -> tuple[to
     probs = torch.empty_like(logits, dtype=torch.float16)
     _, row_entropies, _ = softmax_entropy(logits.view(B * H * S, S), causal=causal, probs=True,
                                           out_probs=probs.view(B * H * S, S))
-    per_batch_entropy = row_entropies.reshape(B, H, S).mean(dim=(1, 2))
+    n = H * S
+    if not 0 < n <= 1 << 17:                          # empty, or long enough for a reduction over many workgroups
+        return probs, row_entropies.reshape(B, H, S).mean(dim=(1, 2))
+    per_batch_entropy = torch.empty(B, dtype=torch.float32, device=logits.device)
+    dev = logits.device
+    with on_device(dev):
+        check(_lib.lib().ee_row_mean(engine_of(dev), ptr(row_entropies), B, n, ptr(per_batch_entropy), stream_of(dev)))
     return probs, per_batch_entropy
 
 
