@@ -702,7 +702,7 @@ static int small_waves(const ee_engine* e, int32_t kind, int64_t M, int64_t N, i
 // routed grid against this one): 8 x 4096 x 4096 19.9 / 12.6, 8 x 2048 x 32000 63 / 43, 64 x 4096 x 14336 54 /
 // 39, 128 x 2048 x 2560 12.3 / 10.7, 128 x 4096 x 14336 57 / 46, 300 x 5632 x 2048 27.1 / 19.4,
 // 300 x 2048 x 2048 13.0 / 10.8; slower at 512 x 2048 x 2048 (13.4 / 14.7), 200 x 4096 x 4096 (20.8 / 22.7),
-// 200 x 4096 x 14336 (58 / 72).  SwiGLU N 11264, K 2048: M 8 25.7 / 22.0, M 64 25.2 / 22.4, M 128 26.0 / 29.6.
+// 200 x 4096 x 14336 (58 / 72).  SwiGLU N 11264, K 2048: M 8 25.7 / 16.4, M 64 25.2 / 18.1, M 128 26.0 / 21.8, M 300 28 / 37.
 // One wave per tile with SwiGLU (98% FP8 rows, M 8: 11.1 us against 15.3 with two) and while that gives at most
 // ~3 workgroups per CU, else two; `dense`: past 4 workgroups per CU of two, the form with half the LDS.
 static int small_routed_waves(const ee_engine* e, int64_t M, int64_t N, int sw, bool& dense) {
@@ -710,7 +710,7 @@ static int small_routed_waves(const ee_engine* e, int64_t M, int64_t N, int sw, 
     const int64_t mt = cdiv(M, 64) + 2, cu = std::max(1, e->cus), n2 = mt * cdiv(N, 32);
     dense = !sw && n2 > 4 * cu;
     if (f >= 0) return std::min(f, sw ? 1 : 2);
-    if (M > (sw ? 64 : 128) && (sw || n2 > 2 * cu)) return 0;
+    if (M > 128 && (sw || n2 > 2 * cu)) return 0;
     return sw || mt * cdiv(N, 16) * 8 <= 25 * cu ? 1 : 2;
 }
 
