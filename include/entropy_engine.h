@@ -303,6 +303,13 @@ int ee_qkv_rope_vt(ee_engine* eng, const void* qkv, int64_t ld, const void* cos_
 int ee_attention_causal(ee_engine* eng, const void* q, const void* k, const void* vt, void* out, int64_t ld_out,
                         float* h, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d, ee_stream_t stream);
 
+/* Both for any S: vt is [B, Hkv, d, S rounded up to 64], zero past S. */
+int ee_qkv_rope_vt_pad(ee_engine* eng, const void* qkv, int64_t ld, const void* cos_t, const void* sin_t, void* q,
+                       void* k, void* vt, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d, float q_scale,
+                       ee_stream_t stream);
+int ee_attention_causal_any(ee_engine* eng, const void* q, const void* k, const void* vt, void* out, int64_t ld_out,
+                            float* h, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d, ee_stream_t stream);
+
 /* Weight preparation: gate_w, up_w fp16 [F, H] and down_w fp16 [H, F] (the
  * nn.Linear layout, EE/test_engine.py:12-14) quantised per output channel as
  * quantize_weights_int8 does (EE/python/dispatch.py:43-48), into the caller's

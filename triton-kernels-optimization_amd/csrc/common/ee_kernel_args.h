@@ -191,14 +191,15 @@ struct EeQkvRopeArgs {
     int64_t ld;
     int32_t B, S, Hq, Hkv, d;
     float q_scale;          // q is stored as fp16(rope(q) * q_scale); 1 stores rope(q)
-    int32_t v_t;            // 1: v is V^T [B, Hkv, d, S], each 16-key group stored as keys 0-3, 8-11, 4-7, 12-15
+    int32_t v_t;            // 0, or V^T's tokens per row (S, or S rounded up to 64: then zero past S): v is
+                            // V^T [B, Hkv, d, v_t], each 16-key group stored as keys 0-3, 8-11, 4-7, 12-15
 };
 
 // Fused causal attention + row entropy (attention.hip), head_dim 64.
 struct EeAttnArgs {
     const uint16_t* q;      // fp16 [B, Hq, S, 64], carrying the 1/sqrt(64) scaling
     const uint16_t* k;      // fp16 [B, Hkv, S, 64]
-    const uint16_t* vt;     // fp16 [B, Hkv, 64, S], key order of eek_qkv_rope's v_t layout
+    const uint16_t* vt;     // fp16 [B, Hkv, 64, S rounded up to 64], eek_qkv_rope's v_t layout
     uint16_t* out;          // fp16 [B*S, ld_out]: token-major, query head h at columns 64h .. 64h + 63
     float* h;               // f32 [B, Hq, S]: entropy of each probability row
     int64_t ld_out;

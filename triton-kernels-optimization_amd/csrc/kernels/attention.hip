@@ -36,8 +36,8 @@
 // order (0-3, 8-11, 4-7, 12-15), so one 16-byte read gives a lane the V^T
 // fragment whose K slots match (written by eek_qkv_rope with v_t set).
 #include "../common/ee_device.h"
+#include "../common/ee_softmax_dev.h"
 
-#define LOG2E 1.4426950408889634f
 #define ATT_STAGE 16384                 // K block 64 x 128 B, then V^T block 64 x 128 B
 
 #define LPTR(p) ((void __attribute__((address_space(3)))*)(p))
@@ -270,8 +270,202 @@ EE_DEV void attn_causal_d64(const EeAttnArgs& a) {
     }
 }
 
+// The same for any S (the launcher's choice where S is not a whole number of key blocks), in two passes
+// over the keys: the row's max and Z, then p = fp16(e^(x - m) / Z) and the softmax kernel's own
+// sums of H.  These are the unfused path's roundings (fp16 scores, fp16 normalised
+// probabilities, H in its cancellation-free form), which such lengths took before: what follows is
+// quantised to 8 bits per row, so probabilities rounded at another scale would move the codes of every
+// row.  The second pass over K costs little: short sequences are bound by the chain of steps, and a step
+// of the first pass is half of one.
+// The last block's K and Q rows past S repeat row S - 1: their keys are masked for every real query (-inf,
+// which no row counts), those queries' results are not stored; V^T is zero past S.
+// Bound by the softmax work of its longest workgroup's steps.  Measured, us, RoPE and attention, unfused (six more
+// launches, scores and probabilities in HBM) / here, 32 query and 4 kv heads: 1 x 300 80 / 29 (the kernel
+// alone 23), 8 x 300 144 / 36, 8 x 511 255 / 49, 2 x 1000 203 / 76, 1 x 4095 1170 / 264.  At 1 x 300 the single-pass
+// form took a few us less and moved the model's logits by 3e-2 of their norm instead of 3e-3.
+template <int W>
+EE_DEV void attn_causal_any_d64(const EeAttnArgs& a) {
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * ATT_STAGE];
+    const int lane = (int)(threadIdx.x & 63), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int r32 = lane & 31, hi = lane >> 5;
+    const int S = a.S, nqb = (S + 63) >> 6, hgroups = a.Hq / W, G = a.Hq / a.Hkv;
+    const int ngrp = a.B * hgroups;
+    const int rank = (int)blockIdx.x / ngrp, hrank = (nqb + 1) >> 1;
+    const int qb = rank < hrank ? nqb - 1 - rank : rank - hrank;
+    const int grp = (int)blockIdx.x % ngrp;
+    const int b = grp / hgroups, hg = grp % hgroups;
+    const int hq = hg * W + wave, hkv = (hg * W) / G;
+    const int q0 = qb << 6, nsteps = qb + 1;
+    const uint32_t Sv = (uint32_t)nqb << 6;           // tokens of a V^T row
+
+    // DMA as in attn_causal_d64; the first pass loads K only.
+    const int64_t kvh = (int64_t)b * a.Hkv + hkv;
+    const uint16_t* kbase = a.k + kvh * S * 64;
+    const uint16_t* vbase = a.vt + kvh * 64 * Sv;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)LPTR(smem);
+    auto issue = [&](int it) {
+        const uint32_t sb = lds0 + (uint32_t)((it & 1) * ATT_STAGE);
+        const bool second = it >= nsteps;
+        const int st = second ? it - nsteps : it;
+#pragma unroll
+        for (int j = 0; j < 16 / W; ++j) {
+            const int i = wave + j * W, g = i & 7, r = 8 * g + (lane >> 3);
+            const uint32_t lc = (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
+            if (i < 8) att_dma16(kbase, (uint32_t)min((st << 6) + r, S - 1) * 128 + lc, sb + (uint32_t)(g * 1024));
+            else if (second) att_dma16(vbase, ((uint32_t)r * Sv + (uint32_t)(st << 6)) * 2 + lc, sb + (uint32_t)(8192 + g * 1024));
+        }
+    };
+    issue(0);
+
+    const uint16_t* qrow = a.q + (((int64_t)b * a.Hq + hq) * S + q0) * 64;
+    u32x4 qf[2][4];
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int dc = 0; dc < 4; ++dc)
+            qf[rb][dc] = *(const u32x4*)(qrow + min(rb * 32 + r32, S - 1 - q0) * 64 + dc * 16 + hi * 8);
+
+    f32x16 o[2][2];
+    float m[2], z[2], t[2], cnt[2], inv[2];
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+        m[rb] = -131008.0f;
+        z[rb] = t[rb] = cnt[rb] = inv[rb] = 0.0f;
+#pragma unroll
+        for (int db = 0; db < 2; ++db) o[rb][db] = f32x16{};
+    }
+
+    for (int it = 0; it < 2 * nsteps; ++it) {
+        ATT_WAITCNT_VM0();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (it + 1 < 2 * nsteps) issue(it + 1);
+        const bool second = it >= nsteps;
+        const bool diag = (second ? it - nsteps : it) == qb;
+        const uint8_t* sk = smem + (it & 1) * ATT_STAGE;
+        const uint8_t* sv = sk + 8192;
+        uint32_t xh[2][2][8];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            u32x4 kf[4];
+#pragma unroll
+            for (int dc = 0; dc < 4; ++dc) kf[dc] = *(const u32x4*)(sk + att_off(kb * 32 + r32, dc * 2 + hi));
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb) {
+                f32x16 acc = f32x16{};
+#pragma unroll
+                for (int dc = 0; dc < 4; ++dc) acc = mma16(kf[dc], qf[rb][dc], acc);
+                if (diag) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (kb * 32 + (r >> 2) * 8 + hi * 4 + (r & 3) > rb * 32 + r32) acc[r] = -INFINITY;
+                }
+#pragma unroll
+                for (int w = 0; w < 8; ++w) xh[rb][kb][w] = pack_f16x2(acc[2 * w], acc[2 * w + 1]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (!second) {
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb) {
+                f16x2 mx2 = f16x2{(f16)-65504.0f, (f16)-65504.0f};
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int w = 0; w < 8; ++w) mx2 = __builtin_elementwise_max(mx2, f16x2_from_bits(xh[rb][kb][w]));
+                float ml = fmaxf((float)mx2.x, (float)mx2.y);
+                ml = fmaxf(ml, __shfl_xor(ml, 32));
+                const float mn = fmaxf(m[rb], ml), negm2 = -mn * LOG2E;
+                float zs = z[rb] * __builtin_amdgcn_exp2f((m[rb] - mn) * LOG2E);
+                m[rb] = mn;
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int w = 0; w < 8; ++w)
+                        zs += __builtin_amdgcn_exp2f(att_l2_lo(xh[rb][kb][w], negm2)) +
+                              __builtin_amdgcn_exp2f(att_l2_hi(xh[rb][kb][w], negm2));
+                z[rb] = zs;
+                if (it + 1 == nsteps) {               // the row is complete: 1 / Z, and the sums of H
+                    inv[rb] = __builtin_amdgcn_rcpf(z[rb] + __shfl_xor(z[rb], 32));
+                    z[rb] = 0.0f;
+                }
+            }
+            continue;
+        }
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+            const float negm = -m[rb];
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int w = 0; w < 8; ++w) {
+                    float e2[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const float s = h ? sub_hi(xh[rb][kb][w], negm) : sub_lo(xh[rb][kb][w], negm);
+                        const float e = __builtin_amdgcn_exp2f(s * LOG2E);
+                        const bool at_max = s == 0.0f;
+                        cnt[rb] += at_max ? 1.0f : 0.0f;
+                        z[rb] += at_max ? 0.0f : e;
+                        t[rb] = fmaf(e, fmaxf(s, -3.0e38f), t[rb]);    // (0 * -inf of a masked key)
+                        e2[h] = e;
+                    }
+                    xh[rb][kb][w] = scale_pack_f16x2(e2[0], e2[1], inv[rb]);
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int db = 0; db < 2; ++db)
+#pragma unroll
+            for (int cc = 0; cc < 4; ++cc) {
+                const u32x4 vf = *(const u32x4*)(sv + att_off(db * 32 + r32, cc * 2 + hi));
+#pragma unroll
+                for (int rb = 0; rb < 2; ++rb) {
+                    const int kb = cc >> 1, w0 = (cc & 1) * 4;
+                    const u32x4 pf = u32x4{xh[rb][kb][w0], xh[rb][kb][w0 + 1], xh[rb][kb][w0 + 2], xh[rb][kb][w0 + 3]};
+                    o[rb][db] = mma16(vf, pf, o[rb][db]);
+                }
+            }
+    }
+
+    ATT_WAITCNT_LGKM0();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    uint8_t* tile = smem + wave * 8192;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+        const float c0 = cnt[rb] + __shfl_xor(cnt[rb], 32), zs = z[rb] + __shfl_xor(z[rb], 32);
+        const float ts = t[rb] + __shfl_xor(t[rb], 32);
+        const int row = q0 + rb * 32 + r32;
+        // no key at the max: the row holds no score above -inf
+        if (hi == 0 && row < S) a.h[((int64_t)b * a.Hq + hq) * S + row] = c0 > 0.0f ? entropy_from(c0, zs, ts) : NAN;
+#pragma unroll
+        for (int db = 0; db < 2; ++db)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int col = db * 32 + q * 8 + hi * 4;
+                *(u32x2*)(tile + att_off(rb * 32 + r32, col >> 3) + ((col >> 2) & 1) * 8) =
+                    u32x2{pack_f16x2(o[rb][db][4 * q], o[rb][db][4 * q + 1]),
+                          pack_f16x2(o[rb][db][4 * q + 2], o[rb][db][4 * q + 3])};
+            }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int row = k * 8 + (lane >> 3), ch = lane & 7;
+        const u32x4 v = *(const u32x4*)(tile + att_off(row, ch));
+        uint16_t* dst = a.out + ((int64_t)b * S + q0 + row) * a.ld_out + (int64_t)hq * 64 + ch * 8;
+        if (q0 + row < S) __builtin_nontemporal_store(v, (u32x4*)dst);
+    }
+}
+
 // One entry per workgroup width W (query heads sharing a kv head per workgroup).
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 eek_attn_causal_d64_w4(EeAttnArgs a) { attn_causal_d64<4>(a); }
 extern "C" __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
 eek_attn_causal_d64_w2(EeAttnArgs a) { attn_causal_d64<2>(a); }
+extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+eek_attn_causal_any_d64_w4(EeAttnArgs a) { attn_causal_any_d64<4>(a); }
+extern "C" __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+eek_attn_causal_any_d64_w2(EeAttnArgs a) { attn_causal_any_d64<2>(a); }

@@ -170,9 +170,10 @@ extern "C" __global__ void __launch_bounds__(EE_BLOCK) eek_qkv_rope(EeQkvRopeArg
     const uint32_t n_qk = T * HH * cpr;
     // v: 16-byte chunks of each token's heads, or with v_t one unit per 16 tokens x
     // 8 d of a kv head, transposed in registers
-    const uint32_t n_v = a.v_t ? (uint32_t)a.B * a.Hkv * (S >> 4) * (d >> 3) : T * a.Hkv * (d >> 3);
+    const uint32_t Sv = (uint32_t)a.v_t;
+    const uint32_t n_v = Sv ? (uint32_t)a.B * a.Hkv * (Sv >> 4) * (d >> 3) : T * a.Hkv * (d >> 3);
     const uint32_t stride = gridDim.x * EE_BLOCK;
-    const uint32_t n_vt = a.v_t ? n_v : 0;
+    const uint32_t n_vt = Sv ? n_v : 0;
     const float q_scale = a.q_scale;
     const bool pow2 = q_scale > 0.0f && (__float_as_uint(q_scale) & 0x007fffffu) == 0 && q_scale >= 0x1p-14f &&
                       q_scale <= 0x1p15f;        // an exact fp16 power of two
@@ -199,18 +200,26 @@ extern "C" __global__ void __launch_bounds__(EE_BLOCK) eek_qkv_rope(EeQkvRopeArg
                                 : a.k + ((int64_t)(b * a.Hkv + (head - a.Hq)) * S + sp) * d;
             *(u32x4*)(dst + 8 * c) = o1;
             *(u32x4*)(dst + h + 8 * c) = o2;
-        } else if (a.v_t) {
-            // V^T [B, Hkv, d, S]: row dd holds v[.., dd] of every token; within each
+        } else if (Sv) {
+            // V^T [B, Hkv, d, Sv]: row dd holds v[.., dd] of every token (zero past S); within each
             // group of 16 tokens the stored order is 0-3, 8-11, 4-7, 12-15 (the
             // K-slot order of the attention kernel's probability fragments).
             const uint32_t iv = i - n_qk;
             const uint32_t c = iv % (d >> 3), r1 = iv / (d >> 3);
-            const uint32_t g = r1 % (S >> 4), bh = r1 / (S >> 4);
+            const uint32_t g = r1 % (Sv >> 4), bh = r1 / (Sv >> 4);
             const uint32_t head = bh % (uint32_t)a.Hkv, b = bh / (uint32_t)a.Hkv;
             const uint16_t* src = a.qkv + (int64_t)(b * S + 16 * g) * a.ld + (HH + head) * d + 8 * c;
             u32x4 x[16];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) x[j] = *(const u32x4*)(src + (int64_t)j * a.ld);
+            for (int j = 0; j < 16; ++j) x[j] = u32x4{};
+            if (16 * g + 16 <= S) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j) x[j] = *(const u32x4*)(src + (int64_t)j * a.ld);
+            } else {                                  // the row's last tokens, or padding
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    if (16 * g + j < S) x[j] = *(const u32x4*)(src + (int64_t)j * a.ld);
+            }
             // stored position p holds token perm(p): chunks of 4 in the order 0, 2, 1, 3
             constexpr int perm[16] = {0, 1, 2, 3, 8, 9, 10, 11, 4, 5, 6, 7, 12, 13, 14, 15};
 #pragma unroll
@@ -220,7 +229,7 @@ extern "C" __global__ void __launch_bounds__(EE_BLOCK) eek_qkv_rope(EeQkvRopeArg
 #pragma unroll
                 for (int k = 0; k < 8; ++k)
                     w[k] = __builtin_amdgcn_perm(x[perm[2 * k + 1]][e >> 1], x[perm[2 * k]][e >> 1], sel);
-                uint16_t* dst = a.v + ((int64_t)(b * a.Hkv + head) * d + 8 * c + e) * S + 16 * g;
+                uint16_t* dst = a.v + ((int64_t)(b * a.Hkv + head) * d + 8 * c + e) * Sv + 16 * g;
                 *(u32x4*)dst = u32x4{w[0], w[1], w[2], w[3]};
                 *(u32x4*)(dst + 8) = u32x4{w[4], w[5], w[6], w[7]};
             }

@@ -15,13 +15,11 @@
 // the row is read from HBM exactly once and the probabilities are written
 // once: 2 bytes in + 2 bytes out per element + 4 bytes of H per row.
 #include "../common/ee_device.h"
+#include "../common/ee_softmax_dev.h"
 
 // 16 bytes of a row, which starts at any multiple of 2 bytes: gfx950 loads and stores them at any
 // address (the compiler emits the same global_load_dwordx4 for either alignment).
 typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
-
-#define LOG2E 1.4426950408889634f
-#define LN2 0.69314718055994531f
 
 // Rows per block for WPR waves per row (the block holds RPB * WPR waves).
 template <int WPR>
@@ -35,35 +33,6 @@ EE_DEV int tier_of(float h, double tl, double th) {
     return d < tl ? 0 : (d < th ? 1 : 2);
 }
 
-// ln x for x >= 1: v_log_f32 (log2, within 1 ulp of the result) times ln 2.
-EE_DEV float ln_ge1(float x) { return __builtin_amdgcn_logf(x) * LN2; }
-// log1p(x) for x >= 0 (Goldberg): u = 1 + x; x ln(u) / (u - 1) with u - 1 exact,
-// which cancels u's rounding, or x where u rounds to 1.  A few ulps relative.
-EE_DEV float log1p_ge0(float x) {
-    const float u = 1.0f + x;
-    return u == 1.0f ? x : ln_ge1(u) * (x * __builtin_amdgcn_rcpf(u - 1.0f));
-}
-// Entropy from the reduced partial sums (see header comment): c0 >= 1 counts the
-// entries at the max, z >= 0, t <= 0, so every term is >= 0; the quotients take
-// v_rcp_f32 (1 ulp).  Within ~1e-6 relative of the libm form (logf, log1pf and
-// IEEE divisions: ~120 dependent instructions, evaluated once per row).
-EE_DEV float entropy_from(float c0, float z, float t) {
-    return ln_ge1(c0) + log1p_ge0(z * __builtin_amdgcn_rcpf(c0)) - t * __builtin_amdgcn_rcpf(c0 + z);
-}
-
-// s = x - m for the low / high fp16 half of a packed word: one v_fma_mix_f32
-// (x * 1 + (-m), a single rounding, the same value as converting x and then
-// subtracting).
-EE_DEV float sub_lo(uint32_t u, float negm) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(u), "v"(negm));
-    return r;
-}
-EE_DEV float sub_hi(uint32_t u, float negm) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(u), "v"(negm));
-    return r;
-}
 // (x - m) log2 e in one v_fma_mix_f32: x * log2e + (-m log2e), one rounding.
 // The waves of a row that hold no entry equal to the max take this form (one
 // instruction per element instead of two); it is within 2^-24 |m log2 e| of
@@ -78,15 +47,6 @@ EE_DEV float sub2_hi(uint32_t u, float l2e, float negml) {
     asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(u), "s"(l2e), "v"(negml));
     return r;
 }
-// fp16(e0 * s) | fp16(e1 * s) << 16, each product rounded once to fp16
-// (v_fma_mixlo_f16 / v_fma_mixhi_f16 with a zero addend).
-EE_DEV uint32_t scale_pack_f16x2(float e0, float e1, float s) {
-    uint32_t r;
-    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(e0), "v"(s));
-    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(r) : "v"(e1), "v"(s));
-    return r;
-}
-
 // A row whose max is within 104 of the lowest fp16 value: -inf entries (masked or padding) clamped to
 // -65504 would count beside it (e^-104 is the first e that is 0 in f32), so the row is moved up by 32768
 // first, exactly (its finite entries are multiples of 32 from -65504 up; -inf stays).

@@ -1219,6 +1219,7 @@ EE_EXPORT int ee_add_rmsnorm_route(ee_engine* eng, const void* x, int64_t ld_x, 
     return launch(eng, std::string("eek_add_rmsnorm_route_") + nc, cdiv(T, EE_BLOCK / 64), 1, EE_BLOCK, ra, stream);
 }
 
+// v_t: 0 v as it is, 1 V^T [.., S], 2 V^T [.., S rounded up to 64], zero past S
 static int qkv_rope_impl(ee_engine* eng, const void* qkv, int64_t ld, const void* cos_t, const void* sin_t,
                          void* q, void* k, void* v, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d,
                          float q_scale, int v_t, ee_stream_t stream) {
@@ -1228,15 +1229,16 @@ static int qkv_rope_impl(ee_engine* eng, const void* qkv, int64_t ld, const void
     if (B < 0 || S < 0 || Hq <= 0 || Hkv <= 0 || d <= 0 || ld < (int64_t)(Hq + 2 * Hkv) * d)
         return fail(EE_ERR_INVALID_ARG, "bad shape or stride");
     if (d % 16 != 0 || ld % 8 != 0) return fail(EE_ERR_UNSUPPORTED, "qkv_rope needs d % 16 == 0 and ld % 8 == 0");
-    if (v_t && S % 16 != 0) return fail(EE_ERR_UNSUPPORTED, "the transposed v layout needs S % 16 == 0");
+    if (v_t == 1 && S % 16 != 0) return fail(EE_ERR_UNSUPPORTED, "the transposed v layout needs S % 16 == 0");
     if (!aligned(qkv, 16) || !aligned(cos_t, 16) || !aligned(sin_t, 16) || !aligned(q, 16) || !aligned(k, 16) ||
         !aligned(v, 16))
         return fail(EE_ERR_INVALID_ARG, "misaligned pointer (16 B)");
-    const int64_t T = (int64_t)B * S;
+    const int64_t T = (int64_t)B * S, Sv = v_t == 2 ? cdiv(S, 64) * 64 : v_t ? S : 0;
     if (T == 0) return EE_OK;
+    if (Sv > INT32_MAX) return fail(EE_ERR_UNSUPPORTED, "qkv_rope: S too large");
     EeQkvRopeArgs a{(const uint16_t*)qkv, (const uint16_t*)cos_t, (const uint16_t*)sin_t, (uint16_t*)q, (uint16_t*)k,
-                    (uint16_t*)v, ld, B, S, Hq, Hkv, d, q_scale, v_t};
-    const int64_t work = T * (Hq + Hkv) * (d / 16) + (v_t ? T / 16 : T) * Hkv * (d / 8);
+                    (uint16_t*)v, ld, B, S, Hq, Hkv, d, q_scale, (int32_t)Sv};
+    const int64_t work = T * (Hq + Hkv) * (d / 16) + (v_t ? B * (Sv / 16) : T) * Hkv * (d / 8);
     if (work >= (int64_t(1) << 31)) return fail(EE_ERR_UNSUPPORTED, "qkv_rope: more than 2^31 work items");
     return launch(eng, "eek_qkv_rope", std::min<int64_t>(cdiv(work, EE_BLOCK), 16384), 1, EE_BLOCK, a, stream);
 }
@@ -1253,14 +1255,21 @@ EE_EXPORT int ee_qkv_rope_vt(ee_engine* eng, const void* qkv, int64_t ld, const 
     return qkv_rope_impl(eng, qkv, ld, cos_t, sin_t, q, k, vt, B, S, Hq, Hkv, d, q_scale, 1, stream);
 }
 
-EE_EXPORT int ee_attention_causal(ee_engine* eng, const void* q, const void* k, const void* vt, void* out,
-                                  int64_t ld_out, float* h, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d,
-                                  ee_stream_t stream) {
+EE_EXPORT int ee_qkv_rope_vt_pad(ee_engine* eng, const void* qkv, int64_t ld, const void* cos_t, const void* sin_t,
+                                 void* q, void* k, void* vt, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d,
+                                 float q_scale, ee_stream_t stream) {
+    return qkv_rope_impl(eng, qkv, ld, cos_t, sin_t, q, k, vt, B, S, Hq, Hkv, d, q_scale, 2, stream);
+}
+
+// any_s: any S, vt padded to whole key blocks; else whole blocks only.
+static int attention_impl(ee_engine* eng, const void* q, const void* k, const void* vt, void* out, int64_t ld_out,
+                          float* h, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d, int any_s,
+                          ee_stream_t stream) {
     if (eng == nullptr || q == nullptr || k == nullptr || vt == nullptr || out == nullptr || h == nullptr)
         return fail(EE_ERR_INVALID_ARG, "NULL argument");
     if (B < 0 || S < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || ld_out < (int64_t)Hq * d)
         return fail(EE_ERR_INVALID_ARG, "bad shape or stride (Hq must be a multiple of Hkv, ld_out >= Hq * d)");
-    if (d != 64 || S % 64 != 0 || ld_out % 8 != 0 || (Hq / Hkv) % 2 != 0)
+    if (d != 64 || (!any_s && S % 64 != 0) || ld_out % 8 != 0 || (Hq / Hkv) % 2 != 0)
         return fail(EE_ERR_UNSUPPORTED, "the fused attention needs head_dim 64, S % 64 == 0, ld_out % 8 == 0 and "
                                         "an even number of query heads per kv head");
     if (!aligned(q, 16) || !aligned(k, 16) || !aligned(vt, 16) || !aligned(out, 16) || !aligned(h, 4))
@@ -1270,8 +1279,27 @@ EE_EXPORT int ee_attention_causal(ee_engine* eng, const void* q, const void* k, 
     const int W = G % 4 == 0 ? 4 : 2;
     EeAttnArgs a{(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)vt, (uint16_t*)out, h, ld_out, B, S, Hq,
                  Hkv, W};
+    // whole key blocks: one pass (32 x 64 heads, 512 tokens: 20 us); else the two-pass kernel, which holds any S
+    // (2 x 2000 tokens 128 us, the unfused path 631)
+    if (S % 64 != 0) {
+        if (S > (1 << 24)) return fail(EE_ERR_UNSUPPORTED, "the fused attention needs S <= 2^24 (32-bit offsets)");
+        return launch(eng, "eek_attn_causal_any_d64_w" + std::to_string(W), (int64_t)B * (Hq / W) * cdiv(S, 64), 1,
+                      64 * W, a, stream);
+    }
     return launch(eng, "eek_attn_causal_d64_w" + std::to_string(W), (int64_t)B * (Hq / W) * (S / 64), 1, 64 * W, a,
                   stream);
+}
+
+EE_EXPORT int ee_attention_causal(ee_engine* eng, const void* q, const void* k, const void* vt, void* out,
+                                  int64_t ld_out, float* h, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d,
+                                  ee_stream_t stream) {
+    return attention_impl(eng, q, k, vt, out, ld_out, h, B, S, Hq, Hkv, d, 0, stream);
+}
+
+EE_EXPORT int ee_attention_causal_any(ee_engine* eng, const void* q, const void* k, const void* vt, void* out,
+                                      int64_t ld_out, float* h, int32_t B, int32_t S, int32_t Hq, int32_t Hkv,
+                                      int32_t d, ee_stream_t stream) {
+    return attention_impl(eng, q, k, vt, out, ld_out, h, B, S, Hq, Hkv, d, 1, stream);
 }
 
 EE_EXPORT int ee_mlp_prepare(ee_engine* eng, const void* gate_w, const void* up_w, const void* down_w, int64_t H,

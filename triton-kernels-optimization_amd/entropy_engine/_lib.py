@@ -84,6 +84,9 @@ SIGNATURES = {
     "ee_qkv_rope_vt": ([_p, _p, _i64, _p, _p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, ctypes.c_float, _p],
                        ctypes.c_int),
     "ee_attention_causal": ([_p, _p, _p, _p, _p, _i64, _p, _i32, _i32, _i32, _i32, _i32, _p], ctypes.c_int),
+    "ee_qkv_rope_vt_pad": ([_p, _p, _i64, _p, _p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, ctypes.c_float, _p],
+                           ctypes.c_int),
+    "ee_attention_causal_any": ([_p, _p, _p, _p, _p, _i64, _p, _i32, _i32, _i32, _i32, _i32, _p], ctypes.c_int),
     "ee_mlp_prepare": ([_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p],
                        ctypes.c_int),
     "ee_mlp_workspace_bytes": ([_i64, _i64, _i64, _i32], _i64),

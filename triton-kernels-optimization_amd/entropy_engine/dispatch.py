@@ -390,9 +390,9 @@ class EntropyGatedLlama:
     one tier per layer.
 
     A token's routing entropy is the mean over heads of its attention-row
-    entropy: the fused attention kernel (attention_causal: scores,
+    entropy: the fused attention kernel (attention_causal_any: scores,
     probabilities and entropies never leave the chip) where its shapes allow
-    (head_dim 64, S % 64 == 0, an even number of query heads per kv head; the
+    (head_dim 64, an even number of query heads per kv head; the
     attribute fused_attention = False turns it off), else the scores, the
     fused softmax+entropy kernel and a product with v.  q/k/v of layer l use layer
     l-1's (layer 0 runs them on the FP16 tier), o/gate/up/down use layer l's,
@@ -546,8 +546,8 @@ class EntropyGatedLlama:
         Hq, Hkv, d = c["heads"], c["kv_heads"], c["head_dim"]
         x = self.p["embed"][input_ids].reshape(T, -1)                    # [T, D] fp16
         cos, sin = self._rope_tables(S, x.device)
-        # the fused attention kernel's shapes (attention_causal); others take the unfused path
-        fused_att = self.fused_attention and d == 64 and S % 64 == 0 and (Hq // Hkv) % 2 == 0
+        # the fused attention kernel's shapes (attention_causal_any); others take the unfused path
+        fused_att = self.fused_attention and d == 64 and (Hq // Hkv) % 2 == 0
         counts_log = []
         self.routes = []
         route_prev = None
@@ -558,8 +558,8 @@ class EntropyGatedLlama:
             # RoPE and the head-major layouts in one pass; q carries the 1/sqrt(d) scaling
             if fused_att:
                 # scores, probabilities and entropies stay on chip; att comes out token-major
-                q, k, vt = K.qkv_rope(qkv, cos, sin, B, S, Hq, Hkv, d, d ** -0.5, v_transposed=True)
-                att, H = K.attention_causal(q, k, vt)
+                q, k, vt = K.qkv_rope(qkv, cos, sin, B, S, Hq, Hkv, d, d ** -0.5, v_padded=True)
+                att, H = K.attention_causal_any(q, k, vt)
             else:
                 q, k, v = K.qkv_rope(qkv, cos, sin, B, S, Hq, Hkv, d, d ** -0.5)
                 att, H = _attention_entropy(q, k, v, 1.0, causal=True)

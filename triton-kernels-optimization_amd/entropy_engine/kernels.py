@@ -527,19 +527,24 @@ def add_rmsnorm_route(x: torch.Tensor, w: torch.Tensor, eps: float, y: torch.Ten
 
 
 def qkv_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, B: int, S: int, Hq: int, Hkv: int, d: int,
-             q_scale: float = 1.0, v_transposed: bool = False):
+             q_scale: float = 1.0, v_transposed: bool = False, v_padded: bool = False):
     """q [B, Hq, S, d], k, v [B, Hkv, S, d] from a fused projection output [B*S, (Hq+2Hkv)*d],
     rotary-embedded (x*cos + rotate_half(x)*sin per fp16 op; cos/sin [S, d]); q scaled by q_scale.
     v_transposed: the third output is attention_causal's vt [B, Hkv, d, S] instead (within each
-    16-token group the order 0-3, 8-11, 4-7, 12-15; see VT_ORDER)."""
+    16-token group the order 0-3, 8-11, 4-7, 12-15; see VT_ORDER).  v_padded: as v_transposed for any S,
+    with S rounded up to 64 in vt and zeros past S: attention_causal_any's."""
     dev = _require_cuda(qkv, cos, sin)
     ld = _rowmajor(qkv, "qkv")
     cos = cos.reshape(S, d).contiguous()
     sin = sin.reshape(S, d).contiguous()
     q = torch.empty((B, Hq, S, d), dtype=torch.float16, device=dev)
     k = torch.empty((B, Hkv, S, d), dtype=torch.float16, device=dev)
-    v = torch.empty((B, Hkv, d, S) if v_transposed else (B, Hkv, S, d), dtype=torch.float16, device=dev)
-    fn = _lib.lib().ee_qkv_rope_vt if v_transposed else _lib.lib().ee_qkv_rope
+    if v_padded:
+        v = torch.empty((B, Hkv, d, (S + 63) // 64 * 64), dtype=torch.float16, device=dev)
+        fn = _lib.lib().ee_qkv_rope_vt_pad
+    else:
+        v = torch.empty((B, Hkv, d, S) if v_transposed else (B, Hkv, S, d), dtype=torch.float16, device=dev)
+        fn = _lib.lib().ee_qkv_rope_vt if v_transposed else _lib.lib().ee_qkv_rope
     with on_device(dev):
         check(fn(engine_of(dev), ptr(qkv), ld, ptr(cos), ptr(sin), ptr(q), ptr(k), ptr(v), B, S, Hq, Hkv, d, float(q_scale),
                  stream_of(dev)))
@@ -555,10 +560,19 @@ def attention_causal(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, out: to
     q [B, Hq, S, 64] (already scaled), k [B, Hkv, S, 64], vt from qkv_rope(v_transposed=True).
     Returns (out [B*S, Hq*64] fp16, token-major, H [B, Hq, S] f32): softmax(q k^T) v over keys <= query,
     and each probability row's Shannon entropy."""
+    return _attention(q, k, vt, out, q.shape[2], _lib.lib().ee_attention_causal)
+
+
+def attention_causal_any(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, out: torch.Tensor | None = None):
+    """attention_causal for any S, with vt from qkv_rope(v_padded=True)."""
+    return _attention(q, k, vt, out, (q.shape[2] + 63) // 64 * 64, _lib.lib().ee_attention_causal_any)
+
+
+def _attention(q, k, vt, out, Sv, fn):
     dev = _require_cuda(q, k, vt, out)
     B, Hq, S, d = q.shape
     Hkv = k.shape[1]
-    if k.shape != (B, Hkv, S, d) or vt.shape != (B, Hkv, d, S):
+    if k.shape != (B, Hkv, S, d) or vt.shape != (B, Hkv, d, Sv):
         raise ValueError(f"shape mismatch: q {tuple(q.shape)}, k {tuple(k.shape)}, vt {tuple(vt.shape)}")
     for t_, n in ((q, "q"), (k, "k"), (vt, "vt")):
         if t_.dtype != torch.float16 or not t_.is_contiguous():
@@ -568,6 +582,5 @@ def attention_causal(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, out: to
     ld_out = _rowmajor(out, "out")
     h = torch.empty((B, Hq, S), dtype=torch.float32, device=dev)
     with on_device(dev):
-        check(_lib.lib().ee_attention_causal(engine_of(dev), ptr(q), ptr(k), ptr(vt), ptr(out), ld_out, ptr(h), B, S, Hq,
-                                             Hkv, d, stream_of(dev)))
+        check(fn(engine_of(dev), ptr(q), ptr(k), ptr(vt), ptr(out), ld_out, ptr(h), B, S, Hq, Hkv, d, stream_of(dev)))
     return out, h
