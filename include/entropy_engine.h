@@ -303,6 +303,11 @@ int ee_qkv_rope_vt(ee_engine* eng, const void* qkv, int64_t ld, const void* cos_
 int ee_attention_causal(ee_engine* eng, const void* q, const void* k, const void* vt, void* out, int64_t ld_out,
                         float* h, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d, ee_stream_t stream);
 
+/* out[t] = sum over l < L of w[l] * counts[l][t], plus extra_fp16 at t = 2 (int64 [3], device): the rows
+ * per tier over a forward's linear calls, from its layers' counts [L, 3]. */
+int ee_route_tally(ee_engine* eng, const int32_t* counts, const int64_t* w, int32_t L, int64_t extra_fp16,
+                   int64_t* out, ee_stream_t stream);
+
 /* Both for any S: vt is [B, Hkv, d, S rounded up to 64], zero past S. */
 int ee_qkv_rope_vt_pad(ee_engine* eng, const void* qkv, int64_t ld, const void* cos_t, const void* sin_t, void* q,
                        void* k, void* vt, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d, float q_scale,

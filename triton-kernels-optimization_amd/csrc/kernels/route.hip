@@ -115,6 +115,18 @@ EE_DEV void route_chunk1(const EeRouteArgs& a, int32_t (*wsum)[3], int tid, int 
     route_place(a, r0, t, pos);
 }
 
+// The rows per tier over a whole forward, one wave per tier.  Bound by its launch: one here where the same
+// sum in tensor operations (stack, widen, multiply, sum, add) is five: a two-layer forward of 8 x 512 tokens
+// 1003 -> 981 us, a one-layer one of 300 tokens 212 -> 202.
+extern "C" __global__ void __launch_bounds__(192) eek_route_tally(EeRouteTallyArgs a) {
+    const int t = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    long long s = 0;
+    for (int l = lane; l < a.L; l += 64) s += (long long)a.counts[3 * l + t] * a.w[l];
+#pragma unroll
+    for (int k = 32; k > 0; k >>= 1) s += __shfl_xor(s, k);
+    if (lane == 0) a.out[t] = s + (t == 2 ? a.extra_fp16 : 0);
+}
+
 // Means of f32 rows (the dispatcher's mean row entropy per batch element): row b of h [rows, seq],
 // one 1024-thread workgroup each, to the b-th f32 of `tier`.  Latency-bound: 8 rows of 16384 2.6 us
 // (torch's reduction 4.9), of 65536 3.9 (7.6); one row of 262144 10.7 (9.6: more workgroups pay there).

@@ -942,6 +942,16 @@ EE_EXPORT int ee_route_heads(ee_engine* eng, const float* h, int32_t B, int32_t 
     return launch(eng, "eek_route", 1, 1, 1024, a, stream);
 }
 
+EE_EXPORT int ee_route_tally(ee_engine* eng, const int32_t* counts, const int64_t* w, int32_t L, int64_t extra_fp16,
+                             int64_t* out, ee_stream_t stream) {
+    if (eng == nullptr || out == nullptr || (L > 0 && (counts == nullptr || w == nullptr)))
+        return fail(EE_ERR_INVALID_ARG, "NULL argument");
+    if (L < 0 || L > INT32_MAX / 3) return fail(EE_ERR_INVALID_ARG, "L out of range");
+    if (!aligned(counts, 4) || !aligned(w, 8) || !aligned(out, 8)) return fail(EE_ERR_INVALID_ARG, "misaligned pointer");
+    EeRouteTallyArgs a{counts, w, out, extra_fp16, L, 0};
+    return launch(eng, "eek_route_tally", 1, 1, 192, a, stream);
+}
+
 EE_EXPORT int ee_row_mean(ee_engine* eng, const float* x, int64_t rows, int32_t n, float* out, ee_stream_t stream) {
     if (eng == nullptr || x == nullptr || out == nullptr) return fail(EE_ERR_INVALID_ARG, "NULL argument");
     if (rows < 0 || n <= 0) return fail(EE_ERR_INVALID_ARG, "need rows >= 0 and n > 0");

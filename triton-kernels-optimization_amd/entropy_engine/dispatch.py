@@ -523,13 +523,15 @@ class EntropyGatedLlama:
         x, xn = K.add_rmsnorm(x, w, self.cfg["eps"], res)
         return x, xn, None
 
-    def _route_heads(self, h: torch.Tensor, counts_log: list):
+    def _route_heads(self, h: torch.Tensor, counts_log: list, counts_all: Optional[torch.Tensor]):
         """Route tokens on the mean over heads of their attention-row entropies
-        h [B, Hq, S] (the mean taken inside the routing kernel)."""
+        h [B, Hq, S] (the mean taken inside the routing kernel); the counts are row
+        len(counts_log) of counts_all [layers, 3]."""
         if self.route_replay is not None:
             idx, counts = self.route_replay[len(counts_log)]
         else:
-            _, idx, counts = K.route_heads(h, self.tau_low, self.tau_high)
+            _, idx, counts = K.route_heads(h, self.tau_low, self.tau_high,
+                                           counts=counts_all[len(counts_log)])
         counts_log.append(counts)
         self.routes.append((idx, counts))
         return idx, counts
@@ -549,6 +551,9 @@ class EntropyGatedLlama:
         # the fused attention kernel's shapes (attention_causal_any); others take the unfused path
         fused_att = self.fused_attention and d == 64 and (Hq // Hkv) % 2 == 0
         counts_log = []
+        replay = self.route_replay is not None
+        counts_all = (torch.empty((c["layers"], 3), dtype=torch.int32, device=x.device)
+                      if gated and not replay else None)
         self.routes = []
         route_prev = None
         res = None                                    # the pending residual branch, added by the next norm
@@ -564,7 +569,7 @@ class EntropyGatedLlama:
                 q, k, v = K.qkv_rope(qkv, cos, sin, B, S, Hq, Hkv, d, d ** -0.5)
                 att, H = _attention_entropy(q, k, v, 1.0, causal=True)
                 att = att.transpose(1, 2).reshape(T, Hq * d)
-            route_cur = self._route_heads(H, counts_log) if gated else None
+            route_cur = self._route_heads(H, counts_log, counts_all) if gated else None
             o = self._linear(att, (l, "o"), route_cur, gated)
             x, xn, xq = self._norm(x, self.p[f"{l}.ln2"], o, route_cur, gated)
             act = self._linear(xn, (l, "gu"), route_cur, gated, swiglu=True, quantized=xq)
@@ -576,7 +581,7 @@ class EntropyGatedLlama:
             # rows per tier over every linear layer (weights in _route_weights); layer
             # 0's q/k/v run on the FP16 tier.  Device ops only: the forward stays
             # capturable as a HIP graph.
-            total = (torch.stack(counts_log).to(torch.int64) * self._route_weights).sum(0)
-            total[2] += 3 * T
-            self.last_fractions = total
+            if replay:
+                counts_all = torch.stack(counts_log).to(torch.int32)
+            self.last_fractions = K.route_tally(counts_all, self._route_weights, 3 * T)
         return logits.view(B, S, -1)

@@ -360,22 +360,40 @@ def route(h: torch.Tensor, tau_low: float, tau_high: float):
     return tier, idx, counts
 
 
-def route_heads(h: torch.Tensor, tau_low: float, tau_high: float):
+def route_heads(h: torch.Tensor, tau_low: float, tau_high: float, counts: torch.Tensor | None = None):
     """route() on the per-token mean over heads of h [B, heads, S] (float32): token
     b * S + s is routed on (h[b, 0, s] + ... + h[b, heads-1, s]) / heads, summed in
-    head order.  Returns (tier int32 [B*S], idx int32 [B*S], counts int32 [3])."""
-    dev = _require_cuda(h)
+    head order.  Returns (tier int32 [B*S], idx int32 [B*S], counts int32 [3]), the counts in `counts` if given."""
+    dev = _require_cuda(h, counts)
     if h.dtype != torch.float32 or h.dim() != 3 or not h.is_contiguous():
         raise TypeError("entropy must be a contiguous [B, heads, S] float32 tensor")
     B, Hh, S = h.shape
     R = B * S
     tier = torch.empty(R, dtype=torch.int32, device=dev)
     idx = torch.empty(R, dtype=torch.int32, device=dev)
-    counts = torch.empty(3, dtype=torch.int32, device=dev)
+    if counts is None:
+        counts = torch.empty(3, dtype=torch.int32, device=dev)
+    elif counts.shape != (3,) or counts.dtype != torch.int32 or not counts.is_contiguous():
+        raise ValueError("counts must be contiguous int32 [3]")
     with on_device(dev):
         check(_lib.lib().ee_route_heads(engine_of(dev), ptr(h), B, Hh, S, float(tau_low), float(tau_high), ptr(tier),
                                         ptr(idx), ptr(counts), stream_of(dev)))
     return tier, idx, counts
+
+
+def route_tally(counts: torch.Tensor, weights: torch.Tensor, extra_fp16: int = 0) -> torch.Tensor:
+    """int64 [3]: sum over l of weights[l] * counts[l] for counts int32 [L, 3] and weights int64 [L],
+    plus extra_fp16 rows of the FP16 tier."""
+    dev = _require_cuda(counts, weights)
+    L = counts.shape[0]
+    if (counts.shape != (L, 3) or counts.dtype != torch.int32 or not counts.is_contiguous()
+            or weights.numel() != L or weights.dtype != torch.int64 or not weights.is_contiguous()):
+        raise ValueError("counts must be contiguous int32 [L, 3], weights contiguous int64 [L]")
+    out = torch.empty(3, dtype=torch.int64, device=dev)
+    with on_device(dev):
+        check(_lib.lib().ee_route_tally(engine_of(dev), ptr(counts), ptr(weights), L, int(extra_fp16), ptr(out),
+                                        stream_of(dev)))
+    return out
 
 
 def row_copy(src: torch.Tensor, idx: torch.Tensor, counts=None, tier: int = 0, scatter: bool = False,
