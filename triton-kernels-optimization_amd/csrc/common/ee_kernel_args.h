@@ -95,21 +95,11 @@ struct EeRoutedGemmArgs {
 // get EE_QUANT_I8_DISPATCH codes, the next counts[1] slots EE_QUANT_F8_ROW codes.
 #define EE_QUANT_ROUTED_I8_F8 16
 
-// Weighted sum of per-layer tier counts (eek_route_tally).
-struct EeRouteTallyArgs {
-    const int32_t* counts;  // [L, 3]
-    const int64_t* w;       // [L]
-    int64_t* out;           // [3]: sum over l of w[l] * counts[l][t], plus extra_fp16 at t = 2
-    int64_t extra_fp16;
-    int32_t L;
-    int32_t pad_;
-};
-
 // Per-row routing: tier + stable partition of row indices.
 struct EeRouteArgs {
     const float* h;         // [rows], or with heads > 1 [rows / seq, heads, seq]: row r = b * seq + s
                             // routes on the mean over heads of h[b, :, s]
-    int32_t* tier;          // [rows] (eek_route_mean: [rows] f32 means)
+    int32_t* tier;          // [rows] (eek_route_mean: [rows] f32 means; eek_route_tally: int64 [3] sums)
     int32_t* idx;           // [rows]: rows of tier 0, then tier 1, then tier 2
     int32_t* counts;        // [3]
     int64_t rows;

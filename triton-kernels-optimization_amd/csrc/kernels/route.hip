@@ -118,13 +118,15 @@ EE_DEV void route_chunk1(const EeRouteArgs& a, int32_t (*wsum)[3], int tid, int 
 // The rows per tier over a whole forward, one wave per tier.  Bound by its launch: one here where the same
 // sum in tensor operations (stack, widen, multiply, sum, add) is five: a two-layer forward of 8 x 512 tokens
 // 1003 -> 981 us, a one-layer one of 300 tokens 212 -> 202.
-extern "C" __global__ void __launch_bounds__(192) eek_route_tally(EeRouteTallyArgs a) {
+extern "C" __global__ void __launch_bounds__(192) eek_route_tally(EeRouteArgs a) {
+    // counts [seq, 3]; h: the layers' weights, int64 [seq]; rows: added to the FP16 tier
+    const int64_t* wt = (const int64_t*)a.h;
     const int t = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
     long long s = 0;
-    for (int l = lane; l < a.L; l += 64) s += (long long)a.counts[3 * l + t] * a.w[l];
+    for (int l = lane; l < a.seq; l += 64) s += (long long)a.counts[3 * l + t] * wt[l];
 #pragma unroll
     for (int k = 32; k > 0; k >>= 1) s += __shfl_xor(s, k);
-    if (lane == 0) a.out[t] = s + (t == 2 ? a.extra_fp16 : 0);
+    if (lane == 0) ((int64_t*)a.tier)[t] = s + (t == 2 ? a.rows : 0);
 }
 
 // Means of f32 rows (the dispatcher's mean row entropy per batch element): row b of h [rows, seq],

@@ -948,7 +948,7 @@ EE_EXPORT int ee_route_tally(ee_engine* eng, const int32_t* counts, const int64_
         return fail(EE_ERR_INVALID_ARG, "NULL argument");
     if (L < 0 || L > INT32_MAX / 3) return fail(EE_ERR_INVALID_ARG, "L out of range");
     if (!aligned(counts, 4) || !aligned(w, 8) || !aligned(out, 8)) return fail(EE_ERR_INVALID_ARG, "misaligned pointer");
-    EeRouteTallyArgs a{counts, w, out, extra_fp16, L, 0};
+    EeRouteArgs a{(const float*)w, (int32_t*)out, nullptr, const_cast<int32_t*>(counts), extra_fp16, 0.0, 0.0, 1, L};
     return launch(eng, "eek_route_tally", 1, 1, 192, a, stream);
 }
 
