@@ -6,6 +6,8 @@
 #include <type_traits>
 
 #include "ee_device.h"
+#define EE_TILE_DIV_FN EE_DEV
+#include "ee_tile_div.h"
 
 // Every epilogue multiply is its own rounded f32 operation, as in the reference.
 #pragma clang fp contract(off)
@@ -210,12 +212,9 @@ EE_DEV bool xcd_share(int n, int& i) {
     return false;
 }
 
-// i / t for tile indices (0 <= i < 2^20, t > 0; a list of that many tiles would be a C of terabytes):
-// (i + 0.5) / t is at least 0.5 / t from an integer and the product below within i / t * 2^-22 of it.  A
-// divide by a count from memory is on the kernel's critical path: an integer division there
-// (~40 dependent instructions) cost 0.4 us per launch.
+// i / t for tile indices of any list (ee_tile_div.h).
 EE_DEV int tile_div(int i, int t) {
-    return __builtin_amdgcn_readfirstlane((int)(((float)i + 0.5f) * __builtin_amdgcn_rcpf((float)t)));
+    return __builtin_amdgcn_readfirstlane(tile_div_rcp(i, t, __builtin_amdgcn_rcpf((float)t)));
 }
 
 // Tile order and the deal of tiles to workgroups (shared by the plain and the
