@@ -1,10 +1,11 @@
 """attention_causal_any and qkv_rope(v_padded=True) at sequence lengths that are not
 whole key blocks, against the unfused path (fp16 scores, softmax_entropy kernel, product with v), which
-served them before, and an fp32 restatement.
+served them before, and restatements in 32 and 64 bits.
 
-Bars: out within 1e-2 of the largest reference value (its probabilities are rounded to fp16, 2^-11 each, at
-another scale than the unfused ones), H within 1e-4 (both from the same fp16 scores in f32;
-a score whose two summation orders round to neighbouring fp16 values moves it by less); padding exact.
+Bars with random inputs: out within 1e-2 of the largest reference value, H within 1e-4.  The probabilities
+are those of the unfused path, but a score whose two summation orders round to neighbouring fp16 values (2^-11
+of |x| <= ~8 apart) moves its probability by up to 2^-8.  With inputs whose scores are exact in any order
+the roundings themselves are held to their bound (test_roundings_of_exact_scores); padding exact.
 """
 import pytest
 import torch
@@ -82,3 +83,43 @@ def test_the_padded_layout_is_checked(ee):
     k = torch.zeros(1, 2, 96, 64, device="cuda", dtype=torch.float16)
     with pytest.raises(ValueError):
         ee.attention_causal_any(q, k, torch.zeros(1, 2, 64, 96, device="cuda", dtype=torch.float16))
+
+
+# scores around 0 and around values where fp16 steps by 0.5, 8 and 32: e^(x - m) and its sum have to come from the
+# difference itself
+@pytest.mark.parametrize("offset,c", [(0, 1), (1000, 1), (10000, 8), (60000, 32)])
+@pytest.mark.parametrize("S", [1, 37, 300, 1001, 2001])
+def test_roundings_of_exact_scores(ee, S, offset, c):
+    """q and k of few bits: every score is exact in f32 in any order, so only p = fp16(e / Z), the
+    sums of out and its store round.  |out - 64 bits| <= 2^-11 (sum p |v| + |out|) + S 2^-25 max |v| (p
+    below fp16's normal range) + f32's share; against the sum of the correctly rounded p, out differs in no more
+    of its last bits than the unfused path's, whose roundings these are."""
+    from entropy_engine.dispatch import _attention_entropy
+    B, Hq, Hkv, d = 1, 4, 2, 64
+    g = torch.Generator(device="cuda").manual_seed(S + offset)
+    tri = lambda n: torch.randint(-1, 2, (S, n, d), device="cuda", generator=g).half()
+    q, k = tri(Hq) * c, tri(Hkv)
+    q[..., 0], k[..., 0] = 8.0, float(offset)              # (q carries a factor 1/8)
+    v = torch.randn(S, Hkv, d, device="cuda", generator=g).half()
+    qkv = torch.cat([q, k, v], dim=1).reshape(S, -1).contiguous()
+    qh, kh, vh, vt = _inputs(ee, B, S, Hq, Hkv, qkv)
+    out, H = ee.attention_causal_any(qh, kh, vt)
+    un_o, un_h = _attention_entropy(qh, kh, vh, 1.0, causal=True)
+    G = Hq // Hkv
+    kr, vr = (t.repeat_interleave(G, dim=1).double() for t in (kh, vh))
+    x = (qh.double() @ kr.transpose(-1, -2).contiguous()).half().double()
+    x = x.masked_fill(~torch.ones(S, S, device="cuda", dtype=torch.bool).tril(), float("-inf"))
+    p = torch.softmax(x, dim=-1)
+    ref, best = p @ vr, (p.half().double() @ vr).half()
+    bar = 2.0 ** -11 * (p @ vr.abs() + ref.abs()) + (S * 2.0 ** -25 + (S // 64 + 64) * 2.0 ** -23) * vr.abs().amax()
+    o = out.view(B, S, Hq, d).transpose(1, 2)
+    assert ((o.double() - ref).abs() <= bar).all()
+    assert torch.equal(o[:, :, 0], vr[:, :, 0].half())                    # one key: p = 1
+    off, off_un = ((t != best).double().mean().item() for t in (o, un_o))
+    assert off <= 1.5 * off_un + 0.01, (off, off_un)
+    s = x - x.amax(dim=-1, keepdim=True)
+    h = torch.logsumexp(s, dim=-1) - (p * s.clamp(min=-1e4)).sum(-1)
+    # f32 sums of a step's 32 terms and of the steps, e to 2^-23 and its argument to 2^-24 |s|
+    tol = (S // 64 + 64) * 2.0 ** -23 * (1 + h)
+    assert ((H.double() - h).abs() <= tol).all()
+    assert ((un_h.double() - h).abs() <= tol).all()

@@ -272,17 +272,23 @@ EE_DEV void attn_causal_d64(const EeAttnArgs& a) {
 
 // The same for any S (the launcher's choice where S is not a whole number of key blocks), in two passes
 // over the keys: the row's max and Z, then p = fp16(e^(x - m) / Z) and the softmax kernel's own
-// sums of H.  These are the unfused path's roundings (fp16 scores, fp16 normalised
-// probabilities, H in its cancellation-free form), which such lengths took before: what follows is
-// quantised to 8 bits per row, so probabilities rounded at another scale would move the codes of every
-// row.  The second pass over K costs little: short sequences are bound by the chain of steps, and a step
+// sums of H.  These are the unfused path's roundings (fp16 scores, e from the exact difference x - m in both
+// passes, fp16 normalised probabilities, H in its cancellation-free form), which such lengths took before:
+// what follows is quantised to 8 bits per row, so probabilities rounded at another scale would move the
+// codes of every row.  (With e from x log2 e + fl(-m log2 e) in the first pass alone, as the single-pass kernel
+// has it where it cancels, Z is off by up to 2^-24 |m|: a last bit of p at |m| = 4000.)  Each step's 32 terms are
+// summed first and then added to the row's sums, as the row kernel's tree does, not one by one over S / 2 keys.
+// The second pass over K costs little: short sequences are bound by the chain of steps, and a step
 // of the first pass is half of one.
 // The last block's K and Q rows past S repeat row S - 1: their keys are masked for every real query (-inf,
 // which no row counts), those queries' results are not stored; V^T is zero past S.
-// Bound by the softmax work of its longest workgroup's steps.  Measured, us, RoPE and attention, unfused (six more
-// launches, scores and probabilities in HBM) / here, 32 query and 4 kv heads: 1 x 300 80 / 29 (the kernel
-// alone 23), 8 x 300 144 / 36, 8 x 511 255 / 49, 2 x 1000 203 / 76, 1 x 4095 1170 / 264.  At 1 x 300 the single-pass
-// form took a few us less and moved the model's logits by 3e-2 of their norm instead of 3e-3.
+// Bound by the softmax work of its longest workgroup's steps.  Measured, us, RoPE and attention from a captured
+// graph, unfused (six more launches, scores and probabilities in HBM) / here, 32 query and 4 kv heads: 1 x 300
+// 45 / 29, 8 x 300 141 / 37, 16 x 130 87 / 28, 2 x 1000 199 / 79, 1 x 4095 1181 / 298; prompts of one or two tokens
+// lose from 64 on (64 x 1 15 / 17, 256 x 1 35 / 46).  The exact difference in the first pass takes 1 to 2% up to
+// 2000 tokens, 6 to 8% of 4000 to 8000.  At 1 x 300 the single-pass form took a few us less and moved the model's
+// logits by 3e-2 of their norm; this one moves them by 2e-3, the share of scores whose f32 sums
+// round to the neighbouring fp16 in the other order.
 template <int W>
 EE_DEV void attn_causal_any_d64(const EeAttnArgs& a) {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * ATT_STAGE];
@@ -376,16 +382,17 @@ EE_DEV void attn_causal_any_d64(const EeAttnArgs& a) {
                     for (int w = 0; w < 8; ++w) mx2 = __builtin_elementwise_max(mx2, f16x2_from_bits(xh[rb][kb][w]));
                 float ml = fmaxf((float)mx2.x, (float)mx2.y);
                 ml = fmaxf(ml, __shfl_xor(ml, 32));
-                const float mn = fmaxf(m[rb], ml), negm2 = -mn * LOG2E;
-                float zs = z[rb] * __builtin_amdgcn_exp2f((m[rb] - mn) * LOG2E);
-                m[rb] = mn;
+                const float mn = fmaxf(m[rb], ml), negm = -mn;
+                float zs[2] = {0.0f, 0.0f};
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                    for (int w = 0; w < 8; ++w)
-                        zs += __builtin_amdgcn_exp2f(att_l2_lo(xh[rb][kb][w], negm2)) +
-                              __builtin_amdgcn_exp2f(att_l2_hi(xh[rb][kb][w], negm2));
-                z[rb] = zs;
+                    for (int w = 0; w < 8; ++w) {
+                        zs[0] += __builtin_amdgcn_exp2f(sub_lo(xh[rb][kb][w], negm) * LOG2E);
+                        zs[1] += __builtin_amdgcn_exp2f(sub_hi(xh[rb][kb][w], negm) * LOG2E);
+                    }
+                z[rb] = fmaf(z[rb], __builtin_amdgcn_exp2f((m[rb] - mn) * LOG2E), zs[0] + zs[1]);
+                m[rb] = mn;
                 if (it + 1 == nsteps) {               // the row is complete: 1 / Z, and the sums of H
                     inv[rb] = __builtin_amdgcn_rcpf(z[rb] + __shfl_xor(z[rb], 32));
                     z[rb] = 0.0f;
@@ -396,6 +403,7 @@ EE_DEV void attn_causal_any_d64(const EeAttnArgs& a) {
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb) {
             const float negm = -m[rb];
+            float zs[2] = {0.0f, 0.0f}, ts[2] = {0.0f, 0.0f}, cs[2] = {0.0f, 0.0f};
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -406,13 +414,16 @@ EE_DEV void attn_causal_any_d64(const EeAttnArgs& a) {
                         const float s = h ? sub_hi(xh[rb][kb][w], negm) : sub_lo(xh[rb][kb][w], negm);
                         const float e = __builtin_amdgcn_exp2f(s * LOG2E);
                         const bool at_max = s == 0.0f;
-                        cnt[rb] += at_max ? 1.0f : 0.0f;
-                        z[rb] += at_max ? 0.0f : e;
-                        t[rb] = fmaf(e, fmaxf(s, -3.0e38f), t[rb]);    // (0 * -inf of a masked key)
+                        cs[h] += at_max ? 1.0f : 0.0f;
+                        zs[h] += at_max ? 0.0f : e;
+                        ts[h] = fmaf(e, fmaxf(s, -3.0e38f), ts[h]);    // (0 * -inf of a masked key)
                         e2[h] = e;
                     }
                     xh[rb][kb][w] = scale_pack_f16x2(e2[0], e2[1], inv[rb]);
                 }
+            cnt[rb] += cs[0] + cs[1];
+            z[rb] += zs[0] + zs[1];
+            t[rb] += ts[0] + ts[1];
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
