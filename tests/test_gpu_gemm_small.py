@@ -132,3 +132,26 @@ def test_small_gemm_choice(ee):
     assert "w8a16" in _last_kernel()
     _opt(1)
     assert torch.equal(_bits(y), _bits(layer(x)))
+
+
+def test_few_rows_pack_the_weight_that_a_captured_call_reads(ee):
+    """A warm-up on decode rows, then a longer call under capture: an eager call before the
+    graph's first replay finds the fp16 weights filled."""
+    from entropy_engine.kernels import gemm_fp16_tier
+    g = torch.Generator(device="cuda").manual_seed(11)
+    codes, scale = ee.quantize_weight_codes((torch.randn(4096, 1024, generator=g, device="cuda") / 32).half())
+    x = torch.randn(1024, 1024, generator=g, device="cuda").half()
+    ref = ee.gemm("fp16", x, ee.PackedWeight(codes, scale).f16)
+    pw = ee.PackedWeight(codes, scale)
+    gemm_fp16_tier(x[:4], pw)
+    assert "w8a16" in _last_kernel()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = gemm_fp16_tier(x, pw)
+    assert "w8a16" not in _last_kernel()
+    assert torch.equal(_bits(gemm_fp16_tier(x, pw)), _bits(ref))
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        assert torch.equal(_bits(y), _bits(ref))

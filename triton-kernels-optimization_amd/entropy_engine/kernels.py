@@ -292,11 +292,14 @@ def gemm(kind: str, a: torch.Tensor, b_nk: torch.Tensor, a_scale=None, b_scale=N
 def gemm_fp16_tier(a: torch.Tensor, pw: PackedWeight, out=None, *, swiglu: bool = False) -> torch.Tensor:
     """The FP16 (W8A16) tier of a packed weight: with few rows from the int8 codes, which the
     small-GEMM kernels dequantise to pw.f16's values in registers (the same bits from half the
-    weight bytes), else from pw.f16."""
+    weight bytes), else from pw.f16.  pw.f16 is packed on the first call whatever its rows: a program that
+    warms up on decode rows may capture a longer call next, and weights packed inside a capture
+    stay unfilled until the graph's first replay."""
+    f16 = pw.f16
     if a.is_cuda and a.shape[0] and pw.i8.data_ptr() % 16 == 0:
         if _lib.lib().ee_gemm_small_waves(engine_of(a.device), _lib.EE_GEMM_W8A16, a.shape[0], pw.N, pw.K, int(swiglu)):
             return gemm("w8a16", a, pw.i8, None, pw.scale, out=out, swiglu=swiglu)
-    return gemm("fp16", a, pw.f16, out=out, swiglu=swiglu)
+    return gemm("fp16", a, f16, out=out, swiglu=swiglu)
 
 
 def _check_gemm_inputs(a, b_int8, b_scale):
