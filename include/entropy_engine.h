@@ -344,6 +344,8 @@ int64_t ee_mlp_workspace_bytes(int64_t M, int64_t H, int64_t F, int32_t routed);
  * The gate|up GEMM writes silu(gate) * up directly (SwiGLU epilogue) when H
  * allows the pipelined kernels (H % 128 == 0); otherwise it stores gate|up and
  * a separate pass applies the activation -- the same bits either way.
+ * gu_* and dn_* are the operands ee_mlp_prepare wrote: the FP16 tier may read gu_f16 / dn_f16 or the int8 codes
+ * and scales they were made from (the same bits).
  * Contract: H % 16 == 0; F % 32 == 0; ld_x multiple of 8; ldo multiple of 4. */
 int ee_mlp_forward(ee_engine* eng, const void* x, int64_t ld_x, int64_t M, int64_t H, int64_t F,
                    const int8_t* gu_i8, const uint8_t* gu_f8, const void* gu_f16, const float* gu_scale,
@@ -404,6 +406,15 @@ int ee_routed_gemm_swiglu(ee_engine* eng, const void* x, int64_t ld_x, int32_t M
                           const int32_t* idx, const int32_t* counts, const int8_t* b_i8, const uint8_t* b_f8,
                           const void* b_f16, const float* b_scale, void* act, int64_t ld_act, const void* codes,
                           const float* scale, ee_stream_t stream);
+/* The four calls above for a weight whose b_f16 is ee_pack_b_f16's of b_i8 and b_scale, by flags: the
+ * SwiGLU form, and codes and scale written beforehand (else they are the workspace).  With few rows the FP16
+ * tier then reads the int8 codes and dequantises them in registers: the same bits from half the weight
+ * bytes.  (The other calls take b_f16 as it is, whatever it holds.) */
+enum { EE_ROUTED_SWIGLU = 1, EE_ROUTED_PREQUANT = 2 };
+int ee_routed_linear_packed(ee_engine* eng, const void* x, int64_t ld_x, int32_t M, int32_t K, int32_t N,
+                            const int32_t* idx, const int32_t* counts, const int8_t* b_i8, const uint8_t* b_f8,
+                            const void* b_f16, const float* b_scale, void* c, int64_t ldc, void* codes, float* scale,
+                            int32_t flags, ee_stream_t stream);
 /* Rows 0..F-1 (gate) and F..2F-1 (up) of src into the interleaved order above
  * (any row payload: int8 codes, e4m3 codes, fp16 weights, or 4-byte scales with
  * row_bytes = 4).  F % 32 == 0; not in place. */

@@ -155,3 +155,30 @@ def test_few_rows_pack_the_weight_that_a_captured_call_reads(ee):
         y.zero_()
         graph.replay()
         assert torch.equal(_bits(y), _bits(ref))
+
+
+@pytest.mark.parametrize("entry", ["linear", "linear_swiglu", "linear_noalloc", "gemm", "gemm_swiglu"])
+@pytest.mark.parametrize("M", [3, 40])
+def test_routed_c_calls_take_b_f16_as_it_is(ee, entry, M):
+    """The C calls do not ask that b_f16 was packed from b_i8 and b_scale: the FP16 rows are b_f16's, with few
+    rows too.  ee_routed_linear_packed does ask it, and refuses flags that it does not know."""
+    from entropy_engine import _lib
+    L, e = _lib.lib(), _lib.engine()
+    K, N, sw = 512, 320, entry.endswith("swiglu")
+    pw, g = _weight(ee, N, K, seed=M)
+    other = torch.randn(N, K, generator=g, device="cuda").half()          # not the codes' values
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    h = torch.where(torch.arange(M, device="cuda") % 3 == 0, 1.0, 3.0)    # INT8 and FP16 rows
+    tier, idx, cnt = ee.route(h, 1.5, 2.5)
+    out = torch.empty(M, N // 2 if sw else N, device="cuda", dtype=torch.float16)
+    codes = torch.zeros(M, K, device="cuda", dtype=torch.uint8)
+    scale = torch.ones(M, device="cuda")
+    head = [e, x.data_ptr(), K, M, K, N, idx.data_ptr(), cnt.data_ptr(), pw.i8.data_ptr(), pw.f8.data_ptr(),
+            other.data_ptr(), pw.scale.data_ptr(), out.data_ptr(), out.shape[1]]
+    ws = [] if entry == "linear_noalloc" else [codes.data_ptr(), scale.data_ptr()]
+    _lib.check(getattr(L, "ee_routed_" + entry)(*head, *ws, _lib.stream_handle()))
+    ref = ee.gemm("fp16", x, other, swiglu=sw)
+    rows = (tier == 2).nonzero().squeeze(1)
+    assert rows.numel() and torch.equal(_bits(out[rows]), _bits(ref[rows]))
+    with pytest.raises(_lib.EngineError, match="flags"):
+        _lib.check(L.ee_routed_linear_packed(*head, codes.data_ptr(), scale.data_ptr(), 4, _lib.stream_handle()))

@@ -976,10 +976,11 @@ EE_EXPORT int ee_row_copy(ee_engine* eng, const void* src, int64_t ld_src_bytes,
     return launch(eng, "eek_row_copy", cdiv(rows, 4), 1, EE_BLOCK, a, stream);
 }
 
+// packed: b_f16 is ee_pack_b_f16 of b_i8 and b_scale, so that a kernel may read either for the FP16 tier.
 static int routed_impl(ee_engine* eng, const void* x, int64_t ld_x, int32_t M, int32_t K, int32_t N,
                        const int32_t* idx, const int32_t* counts, const int8_t* b_i8, const uint8_t* b_f8,
                        const void* b_f16, const float* b_scale, void* c, int64_t ldc, void* ws_codes,
-                       float* ws_scale, int sw, ee_stream_t stream, bool prequant = false) {
+                       float* ws_scale, int sw, ee_stream_t stream, bool prequant = false, bool packed = false) {
     if (eng == nullptr || x == nullptr || idx == nullptr || counts == nullptr || b_i8 == nullptr ||
         b_f8 == nullptr || b_f16 == nullptr || b_scale == nullptr || c == nullptr || ws_codes == nullptr ||
         ws_scale == nullptr)
@@ -1016,7 +1017,8 @@ static int routed_impl(ee_engine* eng, const void* x, int64_t ld_x, int32_t M, i
         ra.mt_max = (int32_t)cdiv(M, 128) + 2;
         ra.f16_w8 = opt(eng, "gemm_variant") == 2;   // the FP16 pipeline ee_gemm picks (same f32 order)
         bool dense = false;
-        if (const int t = small_routed_waves(eng, M, N, sw, dense)) {
+        // (they read the int8 codes for the FP16 tier: only where b_f16 is known to be those codes')
+        if (const int t = packed ? small_routed_waves(eng, M, N, sw, dense) : 0) {
             ra.mt_max = (int32_t)cdiv(M, 64) + 2;
             ra.t[2].b = b_i8;                            // the W8A16 kind: int8 codes and their scales
             ra.t[2].b_scale = b_scale;
@@ -1143,6 +1145,15 @@ EE_EXPORT int ee_routed_gemm_swiglu(ee_engine* eng, const void* x, int64_t ld_x,
                                     int64_t ld_act, const void* codes, const float* scale, ee_stream_t stream) {
     return routed_impl(eng, x, ld_x, M, K, N, idx, counts, b_i8, b_f8, b_f16, b_scale, act, ld_act, (void*)codes,
                        (float*)scale, 1, stream, true);
+}
+
+EE_EXPORT int ee_routed_linear_packed(ee_engine* eng, const void* x, int64_t ld_x, int32_t M, int32_t K, int32_t N,
+                                      const int32_t* idx, const int32_t* counts, const int8_t* b_i8,
+                                      const uint8_t* b_f8, const void* b_f16, const float* b_scale, void* c,
+                                      int64_t ldc, void* codes, float* scale, int32_t flags, ee_stream_t stream) {
+    if (flags & ~(EE_ROUTED_SWIGLU | EE_ROUTED_PREQUANT)) return fail(EE_ERR_INVALID_ARG, "unknown flags");
+    return routed_impl(eng, x, ld_x, M, K, N, idx, counts, b_i8, b_f8, b_f16, b_scale, c, ldc, codes, scale,
+                       flags & EE_ROUTED_SWIGLU ? 1 : 0, stream, (flags & EE_ROUTED_PREQUANT) != 0, true);
 }
 
 EE_EXPORT int ee_interleave_gate_up(ee_engine* eng, const void* src, int64_t ld_src_bytes, void* dst,
@@ -1396,18 +1407,13 @@ EE_EXPORT int ee_mlp_forward(ee_engine* eng, const void* x, int64_t ld_x, int64_
     if (h_rows != nullptr) {
         // one tier per row: route, gate|up routed linear, activation, down routed linear
         if ((rc = ee_route(eng, h_rows, M, tau_low, tau_high, w.tier, w.idx, w.counts, stream))) return rc;
-        if (H % 128 == 0) {                           // gate|up GEMMs write silu(gate) * up directly
-            if ((rc = routed_impl(eng, x, ld_x, m, h, 2 * f, w.idx, w.counts, gu_i8, gu_f8, gu_f16, gu_scale, w.act,
-                                  F, w.codes, w.scale, 1, stream)))
-                return rc;
-        } else {
-            if ((rc = ee_routed_linear(eng, x, ld_x, m, h, 2 * f, w.idx, w.counts, gu_i8, gu_f8, gu_f16, gu_scale,
-                                       w.gu, 2 * F, w.codes, w.scale, stream)))
-                return rc;
-            if ((rc = silu_mul_impl(eng, w.gu, 2 * F, w.act, F, M, F, 1, stream))) return rc;
-        }
-        return ee_routed_linear(eng, w.act, F, m, f, h, w.idx, w.counts, dn_i8, dn_f8, dn_f16, dn_scale, out, ldo,
-                                w.codes, w.scale, stream);
+        const int sw = H % 128 == 0;                  // gate|up GEMMs write silu(gate) * up directly
+        if ((rc = routed_impl(eng, x, ld_x, m, h, 2 * f, w.idx, w.counts, gu_i8, gu_f8, gu_f16, gu_scale,
+                              sw ? (void*)w.act : (void*)w.gu, sw ? F : 2 * F, w.codes, w.scale, sw, stream, false, true)))
+            return rc;
+        if (!sw && (rc = silu_mul_impl(eng, w.gu, 2 * F, w.act, F, M, F, 1, stream))) return rc;
+        return routed_impl(eng, w.act, F, m, f, h, w.idx, w.counts, dn_i8, dn_f8, dn_f16, dn_scale, out, ldo, w.codes,
+                           w.scale, 0, stream, false, true);
     }
     // one tier for the call, by the dispatcher's strict comparisons (EE/python/dispatch.py:74-79)
     const int tier = entropy < tau_low ? EE_TIER_INT8 : (entropy < tau_high ? EE_TIER_FP8 : EE_TIER_FP16);

@@ -35,6 +35,7 @@ EE_TENSOR_WS_FLOATS = 1024
 EE_NOALLOC_MAX_ROWS = 16384              # ee_routed_linear_noalloc's workspace limits
 EE_NOALLOC_MAX_CODE_BYTES = 32 * 1024 * 1024
 EE_GEMM_I8, EE_GEMM_F8, EE_GEMM_F16, EE_GEMM_W8A16 = 0, 1, 2, 3
+EE_ROUTED_SWIGLU, EE_ROUTED_PREQUANT = 1, 2    # flags of ee_routed_linear_packed
 
 _p = ctypes.c_void_p
 _i32 = ctypes.c_int32
@@ -61,6 +62,8 @@ SIGNATURES = {
     "ee_gemm_swiglu": ([_p, _i32, _p, _i64, _p, _i64, _p, _i64, _p, _p, _i32, _i32, _i32, _p, _p, _p, _i32, _p],
                        ctypes.c_int),
     "ee_routed_linear_swiglu": ([_p, _p, _i64, _i32, _i32, _i32, _p, _p, _p, _p, _p, _p, _p, _i64, _p, _p, _p],
+                                ctypes.c_int),
+    "ee_routed_linear_packed": ([_p, _p, _i64, _i32, _i32, _i32, _p, _p, _p, _p, _p, _p, _p, _i64, _p, _p, _i32, _p],
                                 ctypes.c_int),
     "ee_gemm_small_waves": ([_p, _i32, _i64, _i64, _i64, _i32], ctypes.c_int),
     "ee_interleave_gate_up": ([_p, _p, _i64, _p, _i64, _i64, _i64, _p], ctypes.c_int),

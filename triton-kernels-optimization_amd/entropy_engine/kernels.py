@@ -437,17 +437,19 @@ def routed_linear(x: torch.Tensor, pw: PackedWeight, idx: torch.Tensor, counts: 
         if ws_codes.shape != (M, K) or ws_codes.dtype != torch.uint8 or not ws_codes.is_contiguous() \
                 or ws_scale.dtype != torch.float32 or ws_scale.numel() != M:
             raise ValueError("quantized must be (uint8 [M, K] contiguous, float32 [M]) from add_rmsnorm_route")
-        fn = _lib.lib().ee_routed_gemm_swiglu if swiglu else _lib.lib().ee_routed_gemm
+        flags = _lib.EE_ROUTED_PREQUANT
     else:
         if workspace is None:
             workspace = (torch.empty((M, K), dtype=torch.uint8, device=dev),
                          torch.empty(M, dtype=torch.float32, device=dev))
         ws_codes, ws_scale = workspace
-        fn = _lib.lib().ee_routed_linear_swiglu if swiglu else _lib.lib().ee_routed_linear
+        flags = 0
+    if swiglu:
+        flags |= _lib.EE_ROUTED_SWIGLU
     with on_device(dev):
-        check(fn(engine_of(dev), ptr(x), _rowmajor(x, "x"), M, K, N, ptr(idx), ptr(counts), ptr(pw.i8), ptr(pw.f8),
-                 ptr(pw.f16), ptr(pw.scale), ptr(c), _rowmajor(c, "out"), ptr(ws_codes), ptr(ws_scale),
-                 stream_of(dev)))
+        check(_lib.lib().ee_routed_linear_packed(
+            engine_of(dev), ptr(x), _rowmajor(x, "x"), M, K, N, ptr(idx), ptr(counts), ptr(pw.i8), ptr(pw.f8), ptr(pw.f16),
+            ptr(pw.scale), ptr(c), _rowmajor(c, "out"), ptr(ws_codes), ptr(ws_scale), flags, stream_of(dev)))
     return c
 
 
