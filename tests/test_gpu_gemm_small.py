@@ -80,6 +80,24 @@ def test_small_gemm_swiglu_bits(ee, M, K, F, cols):
             assert torch.equal(_bits(ee.gemm("w8a16", x, pw.i8, None, pw.scale, swiglu=True)), _bits(ref)), "w8a16"
 
 
+# the FP8 SwiGLU form of 33 to 64 rows: one buffer of A, K from one stage to several passes over four, with remainders
+@pytest.mark.parametrize("M", [33, 64, 100])
+@pytest.mark.parametrize("K", [128, 256, 512, 640, 2048, 2176])
+def test_fp8_swiglu_of_64_rows(ee, M, K):
+    pw, g = _weight(ee, 192, K, seed=K)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    a, s = ee.quantize_activations(x, "fp8")
+    _, idx, cnt = ee.route(torch.full((M,), 2.0, device="cuda"), 1.5, 2.5)
+    _opt(1)
+    ref = ee.gemm("fp8", a, pw.f8, s, pw.scale, swiglu=True)
+    for cols in (16, 32):
+        _opt(cols)
+        assert torch.equal(_bits(ee.gemm("fp8", a, pw.f8, s, pw.scale, swiglu=True)), _bits(ref))
+        out = torch.full_like(ref, float("nan"))
+        assert torch.equal(_bits(ee.routed_linear(x, pw, idx, cnt, out=out, swiglu=True)), _bits(ref))
+        assert _last_kernel() == "eek_gemm_routed_m64w1_swiglu"
+
+
 def test_small_gemm_int8_accumulators_and_oracle(ee, orc):
     rng = np.random.default_rng(3)
     M, K, N = 21, 1280, 100

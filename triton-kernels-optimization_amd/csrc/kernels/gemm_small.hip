@@ -45,9 +45,12 @@ struct SmallTile {
     static constexpr int ROWS = NI * R;                        // A rows in LDS
     static constexpr int STG = ROWS * BKB;
     static constexpr int CH = CHUNK / STG;                  // stages per chunk
-    // (FP8 SwiGLU at 64 rows holds 64 accumulators: two stages, so that the routed kernel fits 256 registers
-    // and four workgroups a CU: 8 x 2048 x 11264, 20/40/40 % tiers, 19.9 -> 16.4 us)
-    static constexpr int D0 = F8 ? (BJ == 2 ? (NI == 1 ? 4 : 2) : NI == 1 ? 8 : 6) : W8 ? (BJ == 2 ? 8 : 16) : (BJ == 2 ? 6 : 8);
+    // FP8 SwiGLU at 64 rows holds 64 accumulators.  The routed kernel has to fit 256 registers for four workgroups a
+    // CU: four stages of B beside one buffer of A fragments, read just before use (two stages of B beside two buffers
+    // fit too, but hold too few bytes in flight).  us, all rows FP8, 128-tile grid / two stages / this, with the
+    // epilogue's loads below: 33 x 4096 x 4096 16.5 / 20.9 / 17.1, 64 x 4096 x 11264 18.3 / 22.5 / 18.4.
+    static constexpr int NA = F8 && BJ == 2 && NI == 2 ? 1 : 2;
+    static constexpr int D0 = F8 ? (BJ == 2 ? 4 : NI == 1 ? 8 : 6) : W8 ? (BJ == 2 ? 8 : 16) : (BJ == 2 ? 6 : 8);
     static constexpr int D = D0 / CH * CH > 0 ? D0 / CH * CH : CH;   // stages of B in registers: whole chunks
     typedef std::conditional_t<F8, i32x8, i32x4> frag_t;
     typedef std::conditional_t<F8, f32x16, std::conditional_t<F16T, f32x4, i32x4>> acc_t;
@@ -216,9 +219,9 @@ struct SmallTile {
 #pragma unroll
         for (int i = 0; i < D; ++i)
             if (i < nk) load(f[i], i);
-        AStage fa[2];                                          // A, one stage ahead (D is even)
+        AStage fa[NA];                                         // A, one stage ahead with two buffers (D is even)
         barrier();                                             // chunk 0 has landed
-        read(fa[0], smem);
+        if constexpr (NA == 2) read(fa[0], smem);
         // D stages from k0; FULL: all of them are below nk, RELOAD: so are the next D
         auto pass = [&](int k0, auto full, auto reload) {
             constexpr bool FULL = decltype(full)::value, RELOAD = decltype(reload)::value;
@@ -226,7 +229,16 @@ struct SmallTile {
             for (int j = 0; j < BJ; ++j) pb[j] += D * BROW;
 #pragma unroll
             for (int i = 0; i < D; ++i) {
-                if (FULL || k0 + i < nk) {
+                if constexpr (NA == 1) {
+                    if (FULL || k0 + i < nk) {
+                        if (i % CH == 0 && k0 + i > 0) {       // the chunk before has been read, this one has landed
+                            WAITCNT_LGKM0();
+                            barrier();
+                        }
+                        read(fa[0], smem + ((k0 + i) / CH % SM_NC) * CHUNK + i % CH * STG);
+                        compute(f[i], fa[0], acc);
+                    }
+                } else if (FULL || k0 + i < nk) {
                     if ((RELOAD || (FULL && i + 1 < D)) || k0 + i + 1 < nk) {
                         if ((i + 1) % CH == 0) {
                             WAITCNT_LGKM0();                   // this chunk has been read
@@ -250,12 +262,26 @@ struct SmallTile {
 
         // epilogue: lane holds row lr, columns 4 lk .. +3 (FP8: 8 q + 4 lk .. +3) of each block
         constexpr int NQ = F8 ? 4 : 1;
+        // What the stores need from memory, all of it at once: row group by row group under the branch below,
+        // each waited for its own (FP8 SwiGLU 128 x 256 x 2048 7.6 us, now 6.3).
+        int64_t crow[NI];
+        float as[NI];
+        f32x4 bs[BJ][NQ];
 #pragma unroll
         for (int r = 0; r < NI; ++r) {
-            const int m = m0 + r * R + lr;
-            if (m >= M) continue;
-            const int64_t crow = g.c_idx ? (int64_t)g.c_idx[off + m] : (int64_t)m;
-            const float as = F16T ? 0.0f : g.a_scale[off + m];
+            const int m = min(m0 + r * R + lr, M - 1);
+            crow[r] = g.c_idx ? (int64_t)g.c_idx[off + m] : (int64_t)m;
+            as[r] = F16T ? 0.0f : g.a_scale[off + m];
+        }
+        if constexpr (!F16T) {
+#pragma unroll
+            for (int j = 0; j < BJ; ++j)
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) bs[j][q] = *(const f32x4*)(g.b_scale + min(nb[j] + 8 * q + 4 * lk, g.N - 4));
+        }
+#pragma unroll
+        for (int r = 0; r < NI; ++r) {
+            if (m0 + r * R + lr >= M) continue;
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
                 uint32_t o[BJ][2];
@@ -263,22 +289,18 @@ struct SmallTile {
                 for (int j = 0; j < BJ; ++j) {
                     const int n = nb[j] + 8 * q + 4 * lk;
                     float v[4];
-                    f32x4 bs = {0.f, 0.f, 0.f, 0.f};
-                    if constexpr (!F16T) {
-                        if (n < g.N) bs = *(const f32x4*)(g.b_scale + n);
-                    }
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         if constexpr (F16T) v[e] = acc[r][j][4 * q + e];
-                        else v[e] = deq<KIND>(acc[r][j][4 * q + e], as, bs[e]);
+                        else v[e] = deq<KIND>(acc[r][j][4 * q + e], as[r], bs[j][q][e]);
                     }
                     o[j][0] = pack_f16x2(v[0], v[1]);
                     o[j][1] = pack_f16x2(v[2], v[3]);
                     if constexpr (!SW) {
                         if (n < g.N) {                         // N is a multiple of 4
-                            *(u32x2*)(g.c + crow * g.ldc + n) = u32x2{o[j][0], o[j][1]};
+                            *(u32x2*)(g.c + crow[r] * g.ldc + n) = u32x2{o[j][0], o[j][1]};
                             if constexpr (KIND == EE_GEMM_I8) {
-                                if (g.acc) *(i32x4*)(g.acc + crow * g.ldc + n) = acc[r][j];
+                                if (g.acc) *(i32x4*)(g.acc + crow[r] * g.ldc + n) = acc[r][j];
                             }
                         }
                     }
@@ -286,7 +308,7 @@ struct SmallTile {
                 if constexpr (SW) {
                     const int n = cg * R + 8 * q + 4 * lk;
                     if (n < (g.N >> 1))
-                        *(u32x2*)(g.c + crow * g.ldc + n) = u32x2{silu_mul2(o[0][0], o[1][0]), silu_mul2(o[0][1], o[1][1])};
+                        *(u32x2*)(g.c + crow[r] * g.ldc + n) = u32x2{silu_mul2(o[0][0], o[1][0]), silu_mul2(o[0][1], o[1][1])};
                 }
             }
         }
