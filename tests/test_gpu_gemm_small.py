@@ -200,3 +200,14 @@ def test_routed_c_calls_take_b_f16_as_it_is(ee, entry, M):
     assert rows.numel() and torch.equal(_bits(out[rows]), _bits(ref[rows]))
     with pytest.raises(_lib.EngineError, match="flags"):
         _lib.check(L.ee_routed_linear_packed(*head, codes.data_ptr(), scale.data_ptr(), 4, _lib.stream_handle()))
+
+
+def test_few_rows_choice_of_the_codes_for_wide_weights(ee):
+    """From 32 Mi weights on the codes pay up to 128 rows, and up to 256 without SwiGLU where the small tiles pull
+    at most 3/4 of the large tile's bytes; 300 rows of 14336 columns and 700 of 11264 keep the 256-row tiles."""
+    from entropy_engine import _lib
+    L, e, W8 = _lib.lib(), _lib.engine(), _lib.EE_GEMM_W8A16
+    assert L.ee_gemm_small_waves(e, W8, 100, 14336, 4096, 0) > 0
+    assert L.ee_gemm_small_waves(e, W8, 129, 5632, 8192, 0) > 0
+    for M, N, K, sw in [(300, 14336, 4096, 0), (700, 11264, 4096, 0), (384, 11264, 8192, 1), (129, 8192, 4096, 1)]:
+        assert L.ee_gemm_small_waves(e, W8, M, N, K, sw) == 0

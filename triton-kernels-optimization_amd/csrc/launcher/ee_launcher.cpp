@@ -676,7 +676,13 @@ static int small_forced(const ee_engine* e, int sw) {
 //   FP16 against W8A16 codes, K 4096, N 4096: M 4 22.2 / 9.2, M 256 25.1 / 16.4 (0.38); N 14336: M 4
 //     35.3 / 12.9 (0.36), M 128 45.7 / 33.0 (0.75), M 256 47.3 / 62.2 (1.5)
 // W8A16 (int8 codes) also reads half the weight bytes, which counts by itself once the fp16
-// weights leave no room in the Infinity Cache for anything else: N K >= 32 Mi, up to 1.0.
+// weights leave no room in the Infinity Cache for anything else: N K >= 32 Mi, up to 1.0 at up to 128 rows (us, fp16
+// weights on the large tiles / codes here: 100 x 4096 x 14336 42.9 / 34.5, 64 x 1024 x 65536 40.8 / 32.9; but 300 x
+// 4096 x 14336 69.4 / 77.4 and 700 x 4096 x 11264 88 / 129), 0.75 at up to 256 without SwiGLU (129 x 8192 x 5632 54.6 /
+// 39.1; with SwiGLU 129 x 4096 x 8192 32.3 / 34.7).
+// Swept over N 256 to 65536, K 256 to 8192 and 1 to 1024 rows against the kernels chosen without this one, the
+// 256-row ones among them: level or faster but for K >= 4096 at 300 rows or more of N <= 2048 (the ratio 0.5), where the
+// two lie between 5% apart one way and 35% the other.
 static int small_waves(const ee_engine* e, int32_t kind, int64_t M, int64_t N, int64_t K, int sw) {
     const int f = small_forced(e, sw);
     if (f >= 0) return f;
@@ -693,7 +699,8 @@ static int small_waves(const ee_engine* e, int32_t kind, int64_t M, int64_t N, i
             cost = n;
         }
     }
-    const int64_t pct = kind == EE_GEMM_W8A16 && N * K >= (int64_t(32) << 20) ? 100 : M <= 32 ? 75 : 60;
+    const bool half = kind == EE_GEMM_W8A16 && N * K >= (int64_t(32) << 20);
+    const int64_t pct = half && M <= 128 ? 100 : M <= 32 || (half && M <= 256 && !sw) ? 75 : 60;
     return cost * 100 <= large * pct ? best : 0;
 }
 
