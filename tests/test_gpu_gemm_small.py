@@ -211,3 +211,19 @@ def test_few_rows_choice_of_the_codes_for_wide_weights(ee):
     assert L.ee_gemm_small_waves(e, W8, 129, 5632, 8192, 0) > 0
     for M, N, K, sw in [(300, 14336, 4096, 0), (700, 11264, 4096, 0), (384, 11264, 8192, 1), (129, 8192, 4096, 1)]:
         assert L.ee_gemm_small_waves(e, W8, M, N, K, sw) == 0
+
+
+# both sides of each line of the routed choice, on the 256 CUs of an MI355X
+@pytest.mark.parametrize("M,K,N,sw,kernel", [
+    (64, 128, 11008, False, "m64w2_dense"), (65, 128, 11008, False, "eek_gemm_routed"), (65, 128, 2560, False, "m64w1"),
+    (32, 128, 8448, False, "m64w2"), (33, 128, 8448, False, "eek_gemm_routed"), (33, 2048, 8448, False, "m64w2"),
+    (64, 128, 8448, True, "m64w1_swiglu"), (65, 128, 8448, True, "eek_gemm_routed_swiglu"),
+    (128, 128, 8192, True, "m64w1_swiglu"), (129, 128, 8192, True, "eek_gemm_routed_swiglu")])
+def test_routed_choice(ee, M, K, N, sw, kernel):
+    pw, g = _weight(ee, N, K, seed=M)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    _, idx, cnt = ee.route(torch.randint(1, 4, (M,), generator=g, device="cuda").float(), 1.5, 2.5)
+    out = ee.routed_linear(x, pw, idx, cnt, swiglu=sw)
+    assert _last_kernel() == (kernel if kernel.startswith("eek") else "eek_gemm_routed_" + kernel)
+    _opt(1)
+    assert torch.equal(_bits(ee.routed_linear(x, pw, idx, cnt, swiglu=sw)), _bits(out))

@@ -707,18 +707,26 @@ static int small_waves(const ee_engine* e, int32_t kind, int64_t M, int64_t N, i
 // Compute waves of a routed small GEMM, or 0.  The tiers' row counts are on the device; about two M-tiles
 // more than the rows fill are taken to exist.  Measured on 20/40/40 and 1/98/1 % tiers (us, 128-tile
 // routed grid against this one): 8 x 4096 x 4096 19.9 / 12.6, 8 x 2048 x 32000 63 / 43, 64 x 4096 x 14336 54 /
-// 39, 128 x 2048 x 2560 12.3 / 10.7, 128 x 4096 x 14336 57 / 46, 300 x 5632 x 2048 27.1 / 19.4,
-// 300 x 2048 x 2048 13.0 / 10.8; slower at 512 x 2048 x 2048 (13.4 / 14.7), 200 x 4096 x 4096 (20.8 / 22.7),
-// 200 x 4096 x 14336 (58 / 72).  SwiGLU N 11264, K 2048: M 8 25.7 / 16.4, M 64 25.2 / 18.1, M 128 26.0 / 21.8, M 300 28 / 37.
+// 39, 128 x 2048 x 2560 12.3 / 10.7, 300 x 5632 x 2048 27.1 / 19.4, 300 x 2048 x 2048 13.0 / 10.8; slower at 512 x
+// 2048 x 2048 (13.4 / 14.7), 200 x 4096 x 4096 (20.8 / 22.7).  SwiGLU N 11264, K 2048: M 8 25.7 / 16.4, M 64 25.2 / 18.1.
 // One wave per tile with SwiGLU (98% FP8 rows, M 8: 11.1 us against 15.3 with two) and while that gives at most
 // ~3 workgroups per CU, else two; `dense`: past 4 workgroups per CU of two, the form with half the LDS.
-static int small_routed_waves(const ee_engine* e, int64_t M, int64_t N, int sw, bool& dense) {
+// The rule has to hold for every mix of tiers, so it stops where the mixes that gain least lose more than the others
+// gain (us, 128-tile grid / this):
+//   more than 64 rows in more than 4 workgroups per CU of two waves (N > 8192), where two M-tiles read every panel
+//     twice: 100 x 4096 x 32000, one tier 29 / 59, 10/90/0 % 66 / 89, 20/40/40 % 109 / 83; SwiGLU 128 x 4096 x 14336
+//     one tier 21 / 31, 50/50/0 % 22 / 52, 20/40/40 % 40 / 33;
+//   more than 32 rows on two waves at K < 2048 (but for the dense form), whose fixed part shows: 100 x 1024 x 5632
+//     20/40/40 % 9.4 / 11.3, FP16 only 9.7 / 12.1; 64 x 1024 x 8192 20/40/40 % level.
+static int small_routed_waves(const ee_engine* e, int64_t M, int64_t N, int64_t K, int sw, bool& dense) {
     const int f = small_forced(e, sw);
     const int64_t mt = cdiv(M, 64) + 2, cu = std::max(1, e->cus), n2 = mt * cdiv(N, 32);
     dense = !sw && n2 > 4 * cu;
     if (f >= 0) return std::min(f, sw ? 1 : 2);
     if (M > 128 && (sw || n2 > 2 * cu)) return 0;
-    return sw || mt * cdiv(N, 16) * 8 <= 25 * cu ? 1 : 2;
+    if (M > 64 && n2 > 4 * cu) return 0;
+    if (sw || mt * cdiv(N, 16) * 8 <= 25 * cu) return 1;
+    return M > 32 && K < 2048 && !dense ? 0 : 2;
 }
 
 // sw = 1: SwiGLU epilogue (b_nk gate|up interleaved in blocks of 32 rows; c is act [M, N/2]).
@@ -1025,7 +1033,7 @@ static int routed_impl(ee_engine* eng, const void* x, int64_t ld_x, int32_t M, i
         ra.f16_w8 = opt(eng, "gemm_variant") == 2;   // the FP16 pipeline ee_gemm picks (same f32 order)
         bool dense = false;
         // (they read the int8 codes for the FP16 tier: only where b_f16 is known to be those codes')
-        if (const int t = packed ? small_routed_waves(eng, M, N, sw, dense) : 0) {
+        if (const int t = packed ? small_routed_waves(eng, M, N, K, sw, dense) : 0) {
             ra.mt_max = (int32_t)cdiv(M, 64) + 2;
             ra.t[2].b = b_i8;                            // the W8A16 kind: int8 codes and their scales
             ra.t[2].b_scale = b_scale;
