@@ -132,3 +132,15 @@ def test_row_mean(ee, B, H, S):
     ref = h.double().view(B, -1).mean(dim=1)
     # f32 sums of n non-negative values, at most 64 of them in a row
     assert ((ent.double() - ref).abs() <= 64 * 2.0 ** -23 * ref + 1e-30).all()
+
+
+@pytest.mark.parametrize("R,S,causal,group", [(1, 256, False, True), (2559, 257, True, False), (2560, 384, False, True),
+                                              (4095, 385, False, False), (4096, 512, True, True), (2047, 513, False, False),
+                                              (2048, 768, False, True), (2048, 1024, True, True),
+                                              (2048, 1024, False, False), (16384, 1024, False, True),
+                                              (16384, 1025, False, False)])
+def test_softmax_group_choice(ee, R, S, causal, group):
+    """Both sides of each line between one row per wave and several."""
+    x = torch.randn(R, S, device="cuda").half()
+    ee.softmax_entropy(x, causal=causal)
+    assert ("_g16_" in _last_kernel() or "_g32_" in _last_kernel()) == group

@@ -529,13 +529,14 @@ EE_EXPORT int ee_softmax_entropy(ee_engine* eng, const void* x, void* p, float* 
     const bool nt = nt_opt == 2 || (nt_opt == 0 && se_bytes > (int64_t(256) << 20));
     // Rows of 16 to 1024 columns: 4 or 2 rows per wave (eek_softmax_entropy_g*), where the rows then still
     // fill the chip.  Measured, us, one row (or two in turn) per wave against this: [131072, 512] causal 59.9 /
-    // 35.4, all columns 54.0 / 42.4; [40000, 301] 21.6 / 11.7; [16384, 128] 8.6 / 4.1; [4096, 512] 4.3 / 4.15 but
-    // [2048, 512] 3.5 / 4.0, [64, 384] 3.2 / 3.4; two rows per wave: [2048, 1024] causal 4.5 / 4.4, [8192, 768] 8.3 /
-    // 7.3, [16384, 1000] 13.1 / 12.7 but [8192, 1000] 8.5 / 9.0, [512, 777] 4.0 / 4.6.
+    // 35.4, all columns 54.0 / 42.4; [40000, 301] 21.6 / 11.7; [16384, 128] 8.6 / 4.1.  At the lines between: up to 256
+    // columns at any number of rows ([64, 200] 2.76 / 2.78); 384 columns [2048] 3.24 / 3.30, [3000] 3.58 / 3.36, [64] 2.80 /
+    // 3.05; 512 columns [4096] 3.83 / 3.81, [2048] 3.5 / 4.0; two rows per wave: 600 columns [2048] 3.72 / 3.49, 777
+    // causal [2048] 4.63 / 4.40, all columns [16384, 1000] 13.1 / 12.7 but [8192, 1000] 8.5 / 9.0, [512, 777] 4.0 / 4.6.
     // Option "se_group": 0 auto, 1 off, 2 wherever the kernel takes the shape.
     const int64_t g_opt = opt(eng, "se_group");
     const bool g_ok = S >= 16 && S <= 1024 && rows < (int64_t(1) << 31);
-    const bool g_fill = S <= 384 || rows >= (S <= 512 ? 4096 : S <= 768 || causal ? 2048 : 16384);
+    const bool g_fill = S <= 256 || rows >= (S <= 384 ? 2560 : S <= 512 ? 4096 : S <= 768 || causal ? 2048 : 16384);
     if (g_ok && (g_opt == 2 || (g_opt == 0 && g_fill && !opt(eng, "se_wpr") && !opt(eng, "se_rpw")))) {
         const int lpr = S <= 512 ? 16 : 32;
         const std::string name = "eek_softmax_entropy_g" + std::to_string(lpr) + "_v" + std::to_string(cdiv(S, 8 * lpr));
@@ -548,7 +549,8 @@ EE_EXPORT int ee_softmax_entropy(ee_engine* eng, const void* x, void* p, float* 
         // row per wave, 2 or 4 = that many where the variant exists.
         if (wpr == 1 && vpt <= 2) {
             const int64_t f = opt(eng, "se_rpw");
-            // measured at [131072, 512]: 2 rows per wave -8% (causal) to -11%; 4 no better than 2
+            // (automatic below 16 columns only, longer short rows go several to a wave above: [131072, 4] 46.5 / 44.2 us,
+            // [1048576, 15] 366 / 349; 4 rows per wave no better than 2)
             const int rpw = f ? (int)f : (rows >= 32768 ? 2 : 1);
             const std::string rname = "eek_softmax_entropy_v" + std::to_string(vpt) + "_r" + std::to_string(rpw);
             if (rpw > 1 && find_kernel(eng, rname))
