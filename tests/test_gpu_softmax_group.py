@@ -144,3 +144,15 @@ def test_softmax_group_choice(ee, R, S, causal, group):
     x = torch.randn(R, S, device="cuda").half()
     ee.softmax_entropy(x, causal=causal)
     assert ("_g16_" in _last_kernel() or "_g32_" in _last_kernel()) == group
+
+
+@pytest.mark.parametrize("B,H,S,own", [(512, 2, 8, True), (513, 2, 8, False), (513, 64, 64, True), (1030, 1, 1, False)])
+def test_row_mean_of_many_elements(ee, B, H, S, own):
+    """One workgroup per element only where those fill the card no worse than a reduction over rows."""
+    g = torch.Generator(device="cuda").manual_seed(B)
+    x = torch.randn(B, H, S, S, generator=g, device="cuda").half()
+    _, ent = ee.fused_softmax_entropy(x, causal=True)
+    assert ("mean" in _last_kernel()) == own
+    _, h, _ = ee.softmax_entropy(x.view(B * H * S, S), causal=True)
+    ref = h.double().view(B, -1).mean(dim=1)
+    assert ((ent.double() - ref).abs() <= 64 * 2.0 ** -23 * ref + 1e-30).all()
