@@ -123,3 +123,23 @@ def test_roundings_of_exact_scores(ee, S, offset, c):
     tol = (S // 64 + 64) * 2.0 ** -23 * (1 + h)
     assert ((H.double() - h).abs() <= tol).all()
     assert ((un_h.double() - h).abs() <= tol).all()
+
+
+def test_many_prompts_of_one_or_two_tokens_take_the_unfused_path(ee, monkeypatch):
+    """Both sides of the line; the logits are the unfused path's there."""
+    from entropy_engine import dispatch
+    from test_gpu_parity import SMALL_LLAMA
+    m = ee.EntropyGatedLlama.random_init(dict(SMALL_LLAMA, layers=1), seed=3)
+    calls, fused = [], dispatch.K.attention_causal_any
+    monkeypatch.setattr(dispatch.K, "attention_causal_any", lambda *a: calls.append(1) or fused(*a))
+    Hq = SMALL_LLAMA["heads"]
+    for S, line in ((1, 1024 // Hq), (2, 4096 // Hq)):
+        for B in (line, line + 1):
+            ids = torch.randint(0, SMALL_LLAMA["vocab"], (B, S), device="cuda")
+            calls.clear()
+            out = m.forward(ids)
+            assert bool(calls) == (B == line)
+            if B > line:
+                m.fused_attention = False
+                assert torch.equal(out, m.forward(ids))
+                m.fused_attention = True

@@ -548,8 +548,12 @@ class EntropyGatedLlama:
         Hq, Hkv, d = c["heads"], c["kv_heads"], c["head_dim"]
         x = self.p["embed"][input_ids].reshape(T, -1)                    # [T, D] fp16
         cos, sin = self._rope_tables(S, x.device)
-        # the fused attention kernel's shapes (attention_causal_any); others take the unfused path
-        fused_att = self.fused_attention and d == 64 and (Hq // Hkv) % 2 == 0
+        # the fused attention kernel's shapes (attention_causal_any); others take the unfused path.  So do many
+        # prompts of one or two tokens: the kernel takes a workgroup of 64 queries per prompt and 4 heads all the
+        # same (RoPE and attention, 32 heads, us, unfused / fused: 32 x 1 15.1 / 13.2, 48 x 1 15.6 / 16.6, 256 x 1 35 /
+        # 46; 64 x 2 22.5 / 17.4, 128 x 2 27.7 / 28.1, 256 x 2 38 / 47; 256 x 3 57 / 47)
+        fused_att = (self.fused_attention and d == 64 and (Hq // Hkv) % 2 == 0
+                     and not (S <= 2 and B * Hq > 1024 * S * S))
         counts_log = []
         replay = self.route_replay is not None
         counts_all = (torch.empty((c["layers"], 3), dtype=torch.int32, device=x.device)
