@@ -86,6 +86,7 @@ _ARG_STRUCTS = [
     ("eek_gemm4w_routed", "EeRoutedGemmArgs"),
     ("eek_gemm_routed", "EeRoutedGemmArgs"), ("eek_gemm", "EeGemmArgs"),
     ("eek_softmax_entropy", "EeSoftmaxArgs"), ("eek_quant", "EeQuantArgs"), ("eek_absmax_partial", "EeAbsmaxArgs"),
+    ("eek_row_mean", "EeRowMeanArgs"), ("eek_tier_tally", "EeTierTallyArgs"),
     ("eek_route", "EeRouteArgs"), ("eek_transpose_i8", "EeWeightArgs"), ("eek_pack_b", "EeWeightArgs"),
     ("eek_quant_weight", "EeWeightArgs"), ("eek_row_copy", "EeRowCopyArgs"), ("eek_silu_mul", "EeSiluMulArgs"),
     ("eek_interleave_rows", "EeInterleaveArgs"), ("eek_add_rmsnorm_route", "EeRmsNormRouteArgs"),

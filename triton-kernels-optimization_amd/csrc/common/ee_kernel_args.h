@@ -99,7 +99,7 @@ struct EeRoutedGemmArgs {
 struct EeRouteArgs {
     const float* h;         // [rows], or with heads > 1 [rows / seq, heads, seq]: row r = b * seq + s
                             // routes on the mean over heads of h[b, :, s]
-    int32_t* tier;          // [rows] (eek_route_mean: [rows] f32 means; eek_route_tally: int64 [3] sums)
+    int32_t* tier;          // [rows]
     int32_t* idx;           // [rows]: rows of tier 0, then tier 1, then tier 2
     int32_t* counts;        // [3]
     int64_t rows;
@@ -107,6 +107,24 @@ struct EeRouteArgs {
     double tau_high;
     int32_t heads;          // 1: h is per row; 0 (eek_route): tier[] already holds the tiers
     int32_t seq;
+};
+
+// Means of f32 rows, one workgroup each.
+struct EeRowMeanArgs {
+    const float* x;         // [gridDim.x, n]
+    float* out;             // [gridDim.x]
+    int32_t n;
+    int32_t pad;
+};
+
+// Rows per tier over a forward's linear calls.
+struct EeTierTallyArgs {
+    const int32_t* counts;  // [layers, 3]
+    const int64_t* w;       // [layers]: linear calls of the layer
+    int64_t* out;           // [3]: sum of w[l] * counts[l][t], plus extra_fp16 at the FP16 tier
+    int64_t extra_fp16;
+    int32_t layers;
+    int32_t pad;
 };
 
 // Weight preparation (offline, once per layer).

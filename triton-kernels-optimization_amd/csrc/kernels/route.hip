@@ -118,24 +118,22 @@ EE_DEV void route_chunk1(const EeRouteArgs& a, int32_t (*wsum)[3], int tid, int 
 // The rows per tier over a whole forward, one wave per tier.  Bound by its launch: one here where the same
 // sum in tensor operations (stack, widen, multiply, sum, add) is five: a two-layer forward of 8 x 512 tokens
 // 1003 -> 981 us, a one-layer one of 300 tokens 212 -> 202.
-extern "C" __global__ void __launch_bounds__(192) eek_route_tally(EeRouteArgs a) {
-    // counts [seq, 3]; h: the layers' weights, int64 [seq]; rows: added to the FP16 tier
-    const int64_t* wt = (const int64_t*)a.h;
+extern "C" __global__ void __launch_bounds__(192) eek_tier_tally(EeTierTallyArgs a) {
     const int t = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
     long long s = 0;
-    for (int l = lane; l < a.seq; l += 64) s += (long long)a.counts[3 * l + t] * wt[l];
+    for (int l = lane; l < a.layers; l += 64) s += (long long)a.counts[3 * l + t] * a.w[l];
 #pragma unroll
     for (int k = 32; k > 0; k >>= 1) s += __shfl_xor(s, k);
-    if (lane == 0) ((int64_t*)a.tier)[t] = s + (t == 2 ? a.rows : 0);
+    if (lane == 0) a.out[t] = s + (t == 2 ? a.extra_fp16 : 0);
 }
 
-// Means of f32 rows (the dispatcher's mean row entropy per batch element): row b of h [rows, seq],
-// one 1024-thread workgroup each, to the b-th f32 of `tier`.  Latency-bound: 8 rows of 16384 2.6 us
-// (torch's reduction 4.9), of 65536 3.9 (7.6); one row of 262144 10.7 (9.6: more workgroups pay there).
-extern "C" __global__ void __launch_bounds__(1024) eek_route_mean(EeRouteArgs a) {
+// Means of f32 rows (the dispatcher's mean row entropy per batch element): one 1024-thread workgroup
+// each.  Latency-bound.  Per launch in a captured graph, us (torch's reduction): 8 rows of 16384 2.7 (5.0), of 131072
+// 5.7 (11.2); one row of 262144 10.7 (9.6: more workgroups pay there).
+extern "C" __global__ void __launch_bounds__(1024) eek_row_mean(EeRowMeanArgs a) {
     __shared__ float part[16];
-    const int n = a.seq, tid = (int)threadIdx.x;
-    const float* x = a.h + (int64_t)blockIdx.x * n;
+    const int n = a.n, tid = (int)threadIdx.x;
+    const float* x = a.x + (int64_t)blockIdx.x * n;
     float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
     if (((uintptr_t)x & 15) == 0) {
         const int q = n >> 2;
@@ -157,7 +155,7 @@ extern "C" __global__ void __launch_bounds__(1024) eek_route_mean(EeRouteArgs a)
         float t = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) t += part[i];
-        ((float*)a.tier)[blockIdx.x] = t / (float)n;
+        a.out[blockIdx.x] = t / (float)n;
     }
 }
 

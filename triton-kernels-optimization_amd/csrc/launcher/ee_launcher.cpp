@@ -965,8 +965,8 @@ EE_EXPORT int ee_route_tally(ee_engine* eng, const int32_t* counts, const int64_
         return fail(EE_ERR_INVALID_ARG, "NULL argument");
     if (L < 0 || L > INT32_MAX / 3) return fail(EE_ERR_INVALID_ARG, "L out of range");
     if (!aligned(counts, 4) || !aligned(w, 8) || !aligned(out, 8)) return fail(EE_ERR_INVALID_ARG, "misaligned pointer");
-    EeRouteArgs a{(const float*)w, (int32_t*)out, nullptr, const_cast<int32_t*>(counts), extra_fp16, 0.0, 0.0, 1, L};
-    return launch(eng, "eek_route_tally", 1, 1, 192, a, stream);
+    EeTierTallyArgs a{counts, w, out, extra_fp16, L, 0};
+    return launch(eng, "eek_tier_tally", 1, 1, 192, a, stream);
 }
 
 EE_EXPORT int ee_row_mean(ee_engine* eng, const float* x, int64_t rows, int32_t n, float* out, ee_stream_t stream) {
@@ -974,8 +974,8 @@ EE_EXPORT int ee_row_mean(ee_engine* eng, const float* x, int64_t rows, int32_t 
     if (rows < 0 || n <= 0) return fail(EE_ERR_INVALID_ARG, "need rows >= 0 and n > 0");
     if (!aligned(x, 4) || !aligned(out, 4)) return fail(EE_ERR_INVALID_ARG, "misaligned pointer");
     if (rows == 0) return EE_OK;
-    EeRouteArgs a{x, (int32_t*)out, nullptr, nullptr, rows, 0.0, 0.0, 1, n};
-    return launch(eng, "eek_route_mean", rows, 1, 1024, a, stream);
+    EeRowMeanArgs a{x, out, n, 0};
+    return launch(eng, "eek_row_mean", rows, 1, 1024, a, stream);
 }
 
 EE_EXPORT int ee_row_copy(ee_engine* eng, const void* src, int64_t ld_src_bytes, void* dst, int64_t ld_dst_bytes,
