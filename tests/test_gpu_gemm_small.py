@@ -227,3 +227,23 @@ def test_routed_choice(ee, M, K, N, sw, kernel):
     assert _last_kernel() == (kernel if kernel.startswith("eek") else "eek_gemm_routed_" + kernel)
     _opt(1)
     assert torch.equal(_bits(ee.routed_linear(x, pw, idx, cnt, swiglu=sw)), _bits(out))
+
+
+# the form with half the LDS (8 KB chunks: one stage of 33 to 64 rows, one of FP8's 64), which LM heads and wide projections
+# of up to 64 rows take; N with a remainder, K of one stage, five and nine
+@pytest.mark.parametrize("counts", [(1, 0, 0), (3, 4, 1), (16, 17, 31), (0, 0, 64), (0, 64, 0), (64, 0, 0), (5, 40, 19)])
+@pytest.mark.parametrize("K,N", [(128, 32004), (640, 11008), (1152, 11012)])
+def test_dense_routed_bits(ee, counts, K, N):
+    M = sum(counts)
+    pw, g = _weight(ee, N, K, seed=M)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    h = torch.cat([torch.full((c,), t + 1.0) for t, c in enumerate(counts)])[torch.randperm(M)].cuda()
+    _, idx, cnt = ee.route(h, 1.5, 2.5)
+    _opt(1)
+    ref = ee.routed_linear(x, pw, idx, cnt)
+    assert "m64" not in _last_kernel()
+    _opt(0)
+    out = torch.full_like(ref, float("nan"))
+    ee.routed_linear(x, pw, idx, cnt, out=out)
+    assert _last_kernel() == "eek_gemm_routed_m64w2_dense"
+    assert torch.equal(_bits(out), _bits(ref))

@@ -122,6 +122,29 @@ def test_softmax_unaligned_long_rows(ee, orc, R, S, causal):
     assert torch.isnan(out[5:].view(R, S + 2)[:, S:]).all()
 
 
+# the non-temporal loads of the 2-, 4- and 8-wave rows, from rows at any alignment
+@pytest.mark.parametrize("wpr,S", [(2, 4095), (4, 8191), (8, 16383), (8, 20001)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_softmax_unaligned_rows_non_temporal(ee, orc, wpr, S, causal):
+    from entropy_engine import _lib
+    rng = np.random.default_rng(S)
+    X = logits_rows(rng, 9, S)
+    H_ref, P_ref = orc.softmax_entropy(X, causal=causal)
+    _, x = _strided(X, 1, 3)
+    out, p = _strided(np.zeros_like(X), 2, 5)
+    for key, v in ((b"se_wpr", wpr), (b"se_nt", 2)):
+        _lib.check(_lib.lib().ee_engine_set_option(_lib.engine(), key, v))
+    try:
+        _, h, _ = ee.softmax_entropy(x, causal=causal, out_probs=p)
+        assert _last_kernel().endswith("_nt")
+    finally:
+        for key in (b"se_wpr", b"se_nt"):
+            _lib.check(_lib.lib().ee_engine_set_option(_lib.engine(), key, 0))
+    check_entropy(host(h), H_ref)
+    check_probs(host(p), P_ref)
+    assert torch.isnan(out[5:].view(9, S + 2)[:, S:]).all() and torch.isnan(out[:5]).all()
+
+
 @pytest.mark.parametrize("B,H,S", [(1, 1, 1), (3, 5, 33), (2, 7, 64), (8, 32, 512), (2, 3, 171)])
 def test_row_mean(ee, B, H, S):
     g = torch.Generator(device="cuda")
