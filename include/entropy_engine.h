@@ -82,6 +82,8 @@ int ee_engine_destroy(ee_engine* eng);
  * "se_nt" non-temporal loads of the softmax logits in the 2-, 4- and 8-wave
  * row layouts (1 off, 2 on; automatic: on where the logits and probabilities
  * together exceed the 256 MiB Infinity Cache),
+ * "se_group" softmax rows of 16 to 1024 columns several to a wave (1 off, 2 wherever the
+ * kernel takes the shape; automatic: where the rows then fill the chip, unless se_wpr or se_rpw is set),
  * "quant_wpr" waves per quantiser row (1,2,4);
  * "routed_unfused" = 1 makes ee_routed_linear use its five-launch sequence for
  * every K (for comparisons); "gemm_variant" = 1 runs every GEMM on the
@@ -105,7 +107,10 @@ int ee_engine_destroy(ee_engine* eng);
  * "gemm_waves": the pipeline of those 256-row tiles, plain and routed: 8 waves
  * (each a 128 x 64 block) or 4 waves (each a 128 x 128 block, accumulators in
  * AGPRs; tiles of at least two K stages); 0 automatic (4 where it applies).
- * Same bits either way. */
+ * Same bits either way.
+ * "gemm_small": the few-rows GEMM kernels (64-row tiles), plain and ee_routed_linear_packed: 1 off, 16, 32 or
+ * 64 = that many columns per tile at every size (FP8 twice as many; at most 32 with SwiGLU or routed, 16 with both);
+ * automatic by shape.  Any of the gemm_* options above turns the automatic choice off.  Same bits either way. */
 int ee_engine_set_option(ee_engine* eng, const char* key, int64_t value);
 int ee_engine_device(const ee_engine* eng);
 /* Name of the last kernel the calling thread launched through an ee_* entry
@@ -303,17 +308,18 @@ int ee_qkv_rope_vt(ee_engine* eng, const void* qkv, int64_t ld, const void* cos_
 int ee_attention_causal(ee_engine* eng, const void* q, const void* k, const void* vt, void* out, int64_t ld_out,
                         float* h, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d, ee_stream_t stream);
 
-/* out[t] = sum over l < L of w[l] * counts[l][t], plus extra_fp16 at t = 2 (int64 [3], device): the rows
- * per tier over a forward's linear calls, from its layers' counts [L, 3]. */
-int ee_route_tally(ee_engine* eng, const int32_t* counts, const int64_t* w, int32_t L, int64_t extra_fp16,
-                   int64_t* out, ee_stream_t stream);
-
-/* Both for any S: vt is [B, Hkv, d, S rounded up to 64], zero past S. */
+/* ee_qkv_rope_vt and ee_attention_causal for any S: vt is [B, Hkv, d, S rounded up to 64], zero past S.  Where S is
+ * no multiple of 64 the probabilities are the unfused path's fp16(e^(x - m) / Z). */
 int ee_qkv_rope_vt_pad(ee_engine* eng, const void* qkv, int64_t ld, const void* cos_t, const void* sin_t, void* q,
                        void* k, void* vt, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d, float q_scale,
                        ee_stream_t stream);
 int ee_attention_causal_any(ee_engine* eng, const void* q, const void* k, const void* vt, void* out, int64_t ld_out,
                             float* h, int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t d, ee_stream_t stream);
+
+/* out[t] = sum over l < L of w[l] * counts[l][t], plus extra_fp16 at t = 2 (int64 [3], device): the rows
+ * per tier over a forward's linear calls, from its layers' counts [L, 3]. */
+int ee_route_tally(ee_engine* eng, const int32_t* counts, const int64_t* w, int32_t L, int64_t extra_fp16,
+                   int64_t* out, ee_stream_t stream);
 
 /* Weight preparation: gate_w, up_w fp16 [F, H] and down_w fp16 [H, F] (the
  * nn.Linear layout, EE/test_engine.py:12-14) quantised per output channel as

@@ -85,6 +85,17 @@ def test_the_padded_layout_is_checked(ee):
         ee.attention_causal_any(q, k, torch.zeros(1, 2, 64, 96, device="cuda", dtype=torch.float16))
 
 
+def test_what_is_refused_is_named(ee):
+    from entropy_engine import _lib
+    q = torch.zeros(1, 3, 64, 64, device="cuda", dtype=torch.float16)     # an odd number of query heads per kv head
+    k, vt = (torch.zeros(1, 1, 64, 64, device="cuda", dtype=torch.float16) for _ in range(2))
+    with pytest.raises(_lib.EngineError, match="even number") as any_s:
+        ee.attention_causal_any(q, k, vt)
+    with pytest.raises(_lib.EngineError, match="S % 64"):
+        ee.attention_causal(q, k, vt)
+    assert "S % 64" not in str(any_s.value)
+
+
 # scores around 0 and around values where fp16 steps by 0.5, 8 and 32: e^(x - m) and its sum have to come from the
 # difference itself
 @pytest.mark.parametrize("offset,c", [(0, 1), (1000, 1), (10000, 8), (60000, 32)])

@@ -1308,8 +1308,9 @@ static int attention_impl(ee_engine* eng, const void* q, const void* k, const vo
     if (B < 0 || S < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || ld_out < (int64_t)Hq * d)
         return fail(EE_ERR_INVALID_ARG, "bad shape or stride (Hq must be a multiple of Hkv, ld_out >= Hq * d)");
     if (d != 64 || (!any_s && S % 64 != 0) || ld_out % 8 != 0 || (Hq / Hkv) % 2 != 0)
-        return fail(EE_ERR_UNSUPPORTED, "the fused attention needs head_dim 64, S % 64 == 0, ld_out % 8 == 0 and "
-                                        "an even number of query heads per kv head");
+        return fail(EE_ERR_UNSUPPORTED, std::string("the fused attention needs head_dim 64, ") +
+                                            (any_s ? "" : "S % 64 == 0, ") +
+                                            "ld_out % 8 == 0 and an even number of query heads per kv head");
     if (!aligned(q, 16) || !aligned(k, 16) || !aligned(vt, 16) || !aligned(out, 16) || !aligned(h, 4))
         return fail(EE_ERR_INVALID_ARG, "misaligned pointer (q, k, vt, out: 16 B; h: 4 B)");
     if ((int64_t)B * S == 0) return EE_OK;
