@@ -713,13 +713,15 @@ static int small_waves(const ee_engine* e, int32_t kind, int64_t M, int64_t N, i
 // 2048 x 2048 (13.4 / 14.7), 200 x 4096 x 4096 (20.8 / 22.7).  SwiGLU N 11264, K 2048: M 8 25.7 / 16.4, M 64 25.2 / 18.1.
 // One wave per tile with SwiGLU (98% FP8 rows, M 8: 11.1 us against 15.3 with two) and while that gives at most
 // ~3 workgroups per CU, else two; `dense`: past 4 workgroups per CU of two, the form with half the LDS.
-// The rule has to hold for every mix of tiers, so it stops where the mixes that gain least lose more than the others
-// gain (us, 128-tile grid / this):
+// The host does not know the mix of tiers.  Three tiers gain most (the 128-tile grid then takes a second round),
+// one or two least, so the rule stops where those lose more than the others gain (us, 128-tile grid / this):
 //   more than 64 rows in more than 4 workgroups per CU of two waves (N > 8192), where two M-tiles read every panel
 //     twice: 100 x 4096 x 32000, one tier 29 / 59, 10/90/0 % 66 / 89, 20/40/40 % 109 / 83; SwiGLU 128 x 4096 x 14336
-//     one tier 21 / 31, 50/50/0 % 22 / 52, 20/40/40 % 40 / 33;
+//     one tier 21 / 31, 50/50/0 % 21 / 47, 30/30/40 % 45 / 43;
 //   more than 32 rows on two waves at K < 2048 (but for the dense form), whose fixed part shows: 100 x 1024 x 5632
 //     20/40/40 % 9.4 / 11.3, FP16 only 9.7 / 12.1; 64 x 1024 x 8192 20/40/40 % level.
+// What stays on either side of level: SwiGLU of at most 64 rows at N >= 11264, 64 x 4096 x 14336 30/30/40 % 44 / 34
+// but 50/50/0 % 20 / 27; two waves past 128 rows, 300 x 5632 x 2048 20/40/40 % 1.5 x, 76/24/0 % 0.82 x.
 static int small_routed_waves(const ee_engine* e, int64_t M, int64_t N, int64_t K, int sw, bool& dense) {
     const int f = small_forced(e, sw);
     const int64_t mt = cdiv(M, 64) + 2, cu = std::max(1, e->cus), n2 = mt * cdiv(N, 32);
